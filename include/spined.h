@@ -180,7 +180,7 @@ int spined_operator_count_offdiag(const ls_operator *op, uint64_t *out);
 int spined_operator_orbit_method(const ls_operator *op);
 /* Force an orbit method (for parity tests): -1 = automatic. */
 int spined_operator_set_orbit_method(ls_operator *op, int method);
-/* Row schedule of the real matvec kernels: within tiles of 4096 rows the
+/* Row schedule of the matvec kernels: within tiles of 4096 rows the
  * rows are processed in the order of their number of active off-diagonal
  * terms, so the 64 lanes of a wave carry equal work (the sums per row are
  * unchanged).  mode: -1 automatic (on for bases of >= 4096 rows), 0 off,
@@ -194,15 +194,17 @@ int spined_operator_get_schedule(const ls_operator *op);
  * gather-cache matvec keep one lane per row. */
 int spined_operator_set_rows_per_wave(ls_operator *op, int rows);
 int spined_operator_get_rows_per_wave(const ls_operator *op);
-/* Gather cache of a real operator: the target of every term of every row
- * (4 bytes per term, padded per wave: ~74 GB at D = 8.6e8), written once by the orbit and
- * index kernels so that later real single-vector matvecs read it instead of
- * recomputing orbits and searching the index; the sums are identical.
- * mode: -1 automatic (built at a real matvec of a basis of at least 2^20
- * rows when free device memory exceeds it by 4 GiB, and given back whenever
- * a device allocation of the library needs the memory), 0 off, 1 on (built
- * at the next real matvec; an error if it does not fit).  get: 1 while a
- * cache is built.  Changing the row schedule drops the cache. */
+/* Gather cache of an operator: the target of every term of every row (4
+ * bytes per term and 10 per row, padded per wave: ~81 GB at D = 8.6e8),
+ * written once by the orbit and index kernels so that later matvecs read it
+ * instead of recomputing orbits and searching the index; the sums are
+ * identical.
+ * mode: -1 automatic (built when free device memory exceeds it by 4 GiB: at
+ * the first matvec of a basis of at least 2^20 rows or of an operator whose
+ * matrix-free matvec is long, at the second matvec or at a solve otherwise;
+ * given back whenever a device allocation of the library needs the memory),
+ * 0 off, 1 on (built at the next matvec; an error if it does not fit).  get:
+ * 1 while a cache is built.  Changing the row schedule drops the cache. */
 int spined_operator_set_gather_cache(ls_operator *op, int mode);
 int spined_operator_get_gather_cache(const ls_operator *op);
 /* Bucket bits of the bucket index (about 2^bits level-2 buckets of 4 bytes,

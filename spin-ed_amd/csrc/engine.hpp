@@ -63,6 +63,7 @@ struct OrbitTables {
   std::vector<int32_t> h_phases, h_ring_phases;
   int ring_has_rev = 0;
   uint32_t total_terms = 0;
+  uint64_t orbit_cost = 0; // masked shifts and rotations of one generic orbit
   // torus factorisation of the generic orbit (GenericOrbitArgs); l1 = 0: off
   int torus_l1 = 0, torus_l2 = 0;
   std::vector<uint32_t> h_point_elem;
@@ -208,13 +209,17 @@ struct OperatorTables {
 
 void ensure_device(OperatorTables &t);
 
-// Gather cache of a real operator (matvec.hip): the target of every term of
-// every row, written once by the orbit and index kernels, so that later real
+// Gather cache of an operator (matvec.hip): the target of every term of
+// every row, written once by the orbit and index kernels, so that later
 // matvecs read it instead of recomputing orbits and searching the index.
-// Rows in schedule order, one wave per 64 slots; term t of lane l of wave w
-// at entries[woff[w] + 64 t + l] (coalesced).  An entry holds the target
-// index (bits 0..29, all ones: no term), a negative coefficient (bit 30) and
-// a stabiliser ratio other than 1 (bit 31, taken from stab[target]).
+// Rows in schedule order, one wave per 64 slots, woff[w] terms per lane
+// before wave w (woff[waves] the total); a wave's terms in groups of four
+// per lane, the rest one by one (term_pos).  An entry holds the target index
+// (bits 0 .. shift - 1), the class of its coefficient (coefficient of the
+// bond or template times character; below bit 31, or in aux when the two do
+// not fit) and in bit 31 a stabiliser ratio other than 1 (taken from
+// stab[target]).  diag and cnt: the row's diagonal and number of terms, in
+// slot order, so that a cached matvec reads neither states nor bonds.
 struct GatherCache {
   std::mutex mu;
   // set while the holder of mu allocates: a refused allocation reclaims
@@ -222,17 +227,37 @@ struct GatherCache {
   // locking mu a second time
   std::atomic<bool> building{false};
   int request = -1;       // -1 automatic (built when it fits in free memory), 0 off, 1 on
-  bool counted = false;   // woff and total known
+  int calls = 0;          // matvecs before an automatic cache of a small basis
+  bool counted = false;   // classes, woff and total known
   bool built = false;
   uint64_t total = 0;     // entries
+  int32_t phases = 1;     // phase classes: 1 (all trivial), 2 (+-1) or L
+  int32_t nclass = 0, shift = 0;
+  uint32_t imask = 0, cmask = 0;
+  bool in_entry = true;   // classes fit in the entries
+  double one[2] = {0, 0}; // class 0
   DeviceBuffer<uint64_t> woff;
+  DeviceBuffer<double> cls;        // nclass x (re, im)
+  DeviceBuffer<uint16_t> unit_cls; // coefficient class of each unit
   DeviceBuffer<uint32_t> entries;
-  void drop() {           // caller holds mu
+  DeviceBuffer<uint16_t> aux;
+  DeviceBuffer<double> diag;
+  DeviceBuffer<uint16_t> cnt;
+  void release_entries() { // caller holds mu
     built = false;
-    counted = false;
-    total = 0;
     entries.release();
+    aux.release();
+    diag.release();
+    cnt.release();
+  }
+  void drop() {           // caller holds mu
+    release_entries();
+    counted = false;
+    calls = 0;
+    total = 0;
     woff.release();
+    cls.release();
+    unit_cls.release();
   }
 };
 
@@ -244,7 +269,7 @@ struct Operator {
   std::mutex mu;
   spined_stats last_stats{};
   int orbit_method() const; // 0 generic, 1 ring
-  // Row schedule of the real matvec kernels: within every tile of
+  // Row schedule of the matvec kernels: within every tile of
   // kScheduleTile consecutive rows, the rows ordered by their number of
   // active off-diagonal templates, so a wave's lanes carry equal work.
   // sched[i] = offset within the tile of the row processed at slot i.

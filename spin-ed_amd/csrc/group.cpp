@@ -211,6 +211,7 @@ void detect_torus(const Group &g, int n, OrbitTables &t) {
     const uint64_t direct = 2ull * t.total_terms + 2ull * t.nperm;
     const uint64_t torus = 2ull * point_terms + points.size() * (2ull * l1 + 4ull * nt);
     if (torus >= direct) return;
+    t.orbit_cost = torus / 2;
     t.torus_l1 = l1;
     t.torus_l2 = l2;
     t.h_point_elem = points;
@@ -272,6 +273,7 @@ void build_orbit_tables(const Group &g, int n, int spin_inversion, OrbitTables &
     if (ph != 0 && 2 * ph != t.L) t.real_chars = false;
   }
   t.total_terms = static_cast<uint32_t>(t.h_masks.size());
+  t.orbit_cost = t.total_terms;
 
   // Ring detection: every permutation is a rotation p[i] = (i + k) mod n or
   // a reflection p[i] = (c - i) mod n, and all n rotations are present.
@@ -474,7 +476,9 @@ void compile_operator(Operator &op) {
   // other off-diagonal entry -- Heisenberg and XXZ bonds of any strength.
   // Then the diagonal is one select per bond and the (single) active
   // template of an antiparallel bond is the bond itself, in tuple order.
-  t.bonds = t.is_real && t.ntuples > 0;
+  // (Complex sectors too: the gather cache's fill takes the bond form; the
+  // real kernels look at is_real first.)
+  t.bonds = t.ntuples > 0;
   t.h_bond_sites.clear();
   t.h_bond_dp.clear();
   t.h_bond_da.clear();

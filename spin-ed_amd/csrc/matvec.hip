@@ -17,6 +17,8 @@
 // (generic programs or ring run pruning) is a template parameter.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
+#include <map>
 #include <vector>
 
 #include "engine.hpp"
@@ -85,207 +87,370 @@ __global__ void __launch_bounds__(kRowBlock)
 }
 
 // ---- gather cache -----------------------------------------------------------
-constexpr uint32_t kCacheIndex = 0x3FFFFFFFu; // index bits; all ones: no term
-constexpr uint32_t kCacheNeg = 1u << 30;      // negative coefficient
-constexpr uint32_t kCacheRatio = 1u << 31;    // sqrt(|Stab target| / |Stab row|) != 1
+// Active units (exchange bonds or templates) of a row, over any number of
+// them.
+template <bool BONDS>
+__device__ inline uint32_t row_count(const OpArgs &o, const BondArgs &bd, uint64_t r) {
+  uint32_t c = 0;
+  if constexpr (BONDS) {
+    for (int t = 0; t < bd.nbonds; ++t) {
+      const uint32_t s = bd.sites[t];
+      const uint32_t anti = static_cast<uint32_t>((r >> (s & 0xffu)) ^ (r >> (s >> 8))) & 1u;
+      c += bd.o[t] != 0.0 ? anti : 0u;
+    }
+  } else {
+    for (int t = 0; t < o.ntuples; ++t) {
+      const uint32_t *rg = o.range + o.tuple_off[t] + t +
+                           local_state(o.tuple_sites[t], static_cast<int>(o.tuple_n[t]), r);
+      c += rg[1] - rg[0];
+    }
+  }
+  return c;
+}
+
+// Diagonal of a row, summed in tuple order as the matrix-free kernels do.
+template <bool BONDS>
+__device__ inline double2 row_diag(const OpArgs &o, const BondArgs &bd, uint64_t r) {
+  double re = 0.0, im = 0.0;
+  if constexpr (BONDS) {
+    for (int t = 0; t < bd.nbonds; ++t) {
+      const uint32_t s = bd.sites[t];
+      re += (((r >> (s & 0xffu)) ^ (r >> (s >> 8))) & 1u) ? bd.da[t] : bd.dp[t];
+    }
+  } else {
+    for (int t = 0; t < o.ntuples; ++t) {
+      const int a = local_state(o.tuple_sites[t], static_cast<int>(o.tuple_n[t]), r);
+      re += o.diag_re[o.tuple_off[t] + a];
+      im += o.diag_im[o.tuple_off[t] + a];
+    }
+  }
+  return make_double2(re, im);
+}
+
+// Active units base .. base + 64 NW - 1 of a row, one bit each.
+template <int NW, bool BONDS>
+__device__ inline void row_active(const OpArgs &o, const BondArgs &bd, uint64_t r, int base,
+                                  uint64_t (&act)[NW]) {
+#pragma unroll
+  for (int w = 0; w < NW; ++w) act[w] = 0;
+  if constexpr (BONDS) {
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const int tb = base + 64 * w;
+      const int te = bd.nbonds < tb + 64 ? bd.nbonds : tb + 64;
+      for (int t = tb; t < te; ++t) {
+        const uint32_t s = bd.sites[t];
+        const uint64_t anti = ((r >> (s & 0xffu)) ^ (r >> (s >> 8))) & 1u;
+        if (bd.o[t] != 0.0) act[w] |= anti << (t - tb);
+      }
+    }
+  } else {
+    const uint32_t lo = static_cast<uint32_t>(base), hi = lo + 64u * NW;
+    for (int t = 0; t < o.ntuples; ++t) {
+      const uint32_t *rg = o.range + o.tuple_off[t] + t +
+                           local_state(o.tuple_sites[t], static_cast<int>(o.tuple_n[t]), r);
+      const uint32_t b = rg[0] > lo ? rg[0] : lo, e = rg[1] < hi ? rg[1] : hi;
+      if (b < e) mark_range<NW>(act, b - lo, e - lo);
+    }
+  }
+}
+
+// Where term t of a lane lies in its wave's entries: the wave's terms in
+// groups of four per lane (one 16-byte load each), the last T mod 4 one by
+// one (no padding beyond the wave's busiest row).
+__device__ inline uint64_t term_pos(uint32_t t, uint32_t T, uint32_t lane) {
+  const uint32_t full = T & ~3u;
+  return t < full ? (static_cast<uint64_t>(t >> 2) * 256 + 4 * lane + (t & 3u))
+                  : static_cast<uint64_t>(t) * 64 + lane;
+}
 
 // Terms of the busiest row of each wave (one wave = 64 slots).
-template <int NW, bool BONDS>
+template <bool BONDS>
 __global__ void __launch_bounds__(kRowBlock)
     cache_count_kernel(OpArgs o, BondArgs bd, const uint64_t *__restrict__ reps, uint64_t D,
                        const uint16_t *__restrict__ sched, uint32_t *__restrict__ wave_terms) {
   const uint64_t slot = static_cast<uint64_t>(blockIdx.x) * kRowBlock + threadIdx.x;
   uint32_t c = 0;
-  if (slot < D) {
-    uint64_t act[NW];
-    (void)row_pass_a<NW, BONDS>(o, bd, reps[scheduled_row(sched, slot)], act);
-#pragma unroll
-    for (int w = 0; w < NW; ++w) c += static_cast<uint32_t>(__popcll(act[w]));
-  }
+  if (slot < D) c = row_count<BONDS>(o, bd, reps[scheduled_row(sched, slot)]);
   for (int off = 32; off > 0; off >>= 1) c = max(c, static_cast<uint32_t>(__shfl_xor(c, off, 64)));
   if (threadIdx.x == 0) wave_terms[blockIdx.x] = c;
 }
 
+// What the cached kernels read (GatherCache; engine.hpp has the layout).
+struct CacheArgs {
+  const uint64_t *__restrict__ woff;
+  const uint32_t *__restrict__ entries;
+  const uint16_t *__restrict__ aux;  // class of each term when it has no room in the entry
+  const double *__restrict__ diag;   // per slot: one double, or two (re, im)
+  const uint16_t *__restrict__ cnt;  // per slot
+  const double *__restrict__ cls;    // nclass x (re, im)
+  int32_t nclass;
+  int32_t shift;                     // class = (entry >> shift) & cmask
+  uint32_t imask, cmask;
+};
+
 // Entries of every term, in the order and with the orbits and lookups of
-// gather_row_real.
-template <int METHOD, int NW, bool BONDS>
-__global__ void __launch_bounds__(kRowBlock)
+// gather_row_real; units beyond 64 NW in further rounds.  unit_cls: the
+// coefficient class of each unit; phases: phase classes, 1 (all characters
+// trivial), 2 (+-1) or L; CLS: more than one coefficient.  The outputs are arguments of their own: restrict
+// does not hold inside a struct, and without it the group's programs are
+// read by vector loads instead of scalar ones (2x the time on a 384-element
+// group).
+template <int METHOD, int NW, bool BONDS, bool CLS>
+__global__ void __launch_bounds__(kRowBlock, 7)
     cache_fill_kernel(OpArgs o, BondArgs bd, GenericOrbitArgs ga, RingOrbitArgs ra, IndexArgs ix,
                       const uint32_t *__restrict__ stab, uint64_t D,
                       const uint16_t *__restrict__ sched, const uint64_t *__restrict__ woff,
-                      uint32_t *__restrict__ entries) {
+                      const uint16_t *__restrict__ unit_cls, int32_t phases, int32_t shift,
+                      int32_t complex_diag, uint32_t *__restrict__ entries,
+                      uint16_t *__restrict__ aux, double *__restrict__ diag,
+                      uint16_t *__restrict__ cnt) {
   ix = index_for_method<METHOD>(ix);
+  const int units = BONDS ? bd.nbonds : o.ntemplates;
+  __shared__ uint16_t s_cls[CLS ? 64 * NW : 1];
+  if constexpr (CLS) {
+    if (units <= 64 * NW)
+      for (int j = threadIdx.x; j < units; j += kRowBlock) s_cls[j] = unit_cls[j];
+    __syncthreads();
+  }
   const uint64_t slot = static_cast<uint64_t>(blockIdx.x) * kRowBlock + threadIdx.x;
   if (slot >= D) return;
   const uint64_t i = scheduled_row(sched, slot);
   const uint64_t r = ix.reps[i];
-  uint64_t act[NW];
-  (void)row_pass_a<NW, BONDS>(o, bd, r, act);
+  const double2 dg = row_diag<BONDS>(o, bd, r);
+  if (complex_diag) {
+    diag[2 * slot] = dg.x;
+    diag[2 * slot + 1] = dg.y;
+  } else {
+    diag[slot] = dg.x;
+  }
   const RowOrbit<METHOD, BONDS> rob(ra, bd, r);
   const int32_t si = static_cast<int32_t>(stab[i]);
-  uint32_t *out = entries + woff[blockIdx.x] * 64 + threadIdx.x;
+  const uint64_t w0 = woff[blockIdx.x];
+  const uint32_t T = static_cast<uint32_t>(woff[blockIdx.x + 1] - w0);
+  uint32_t *out = entries + w0 * 64;
   // generic groups with trivial characters: the orbit minimum alone (no
   // phase can differ), |Stab| of the target from the basis' entry
   const bool min_only = METHOD == 0 && ga.trivial;
-  auto entry = [&](int64_t k, const OrbitResult &orb) {
-    if (k < 0) return kCacheIndex;
-    const int32_t cnt = min_only ? static_cast<int32_t>(stab[k]) : orb.count;
-    return static_cast<uint32_t>(k) | (orb.phase != 0 ? kCacheNeg : 0u) |
-           (cnt != si ? kCacheRatio : 0u);
-  };
-  auto orbit_of = [&](int j) {
-    if (min_only)
-      return OrbitResult{orbit_min_generic(ga, r ^ (BONDS ? bd.flip[j] : o.flip[j])), 0, 0, true};
-    return rob.orbit(o, bd, ga, ra, r, j);
-  };
-  int t = 0;
-  while (any_set<NW>(act)) {
-    const int ja = pop_first<NW>(act);
-    const int jb = pop_first<NW>(act);
-    const OrbitResult oa = orbit_of(ja);
-    OrbitResult ob{0, 0, 0, false};
-    if (jb >= 0) ob = orbit_of(jb);
-    int64_t ka, kb;
-    find_index2(ix, oa.rep, oa.valid, ob.rep, ob.valid, ka, kb);
-    out[64 * static_cast<uint64_t>(t++)] = entry(ka, oa);
-    if (jb >= 0) out[64 * static_cast<uint64_t>(t++)] = entry(kb, ob);
-  }
-}
-
-// Real matvec from the gather cache: the sums of matvec_real_kernel (same
-// terms, coefficients and order) without orbits or index searches.
-template <int NW, bool BONDS, class XT, class YT>
-__global__ void __launch_bounds__(kRowBlock)
-    matvec_cached_kernel(OpArgs o, BondArgs bd, RatioArgs rt, const uint64_t *__restrict__ reps,
-                         const uint32_t *__restrict__ stab, uint64_t D,
-                         const XT *__restrict__ x, YT *__restrict__ y,
-                         const uint16_t *__restrict__ sched, const uint64_t *__restrict__ woff,
-                         const uint32_t *__restrict__ entries) {
-  __shared__ double so[BONDS ? 64 * NW : 1];
-  if constexpr (BONDS) {
-    for (int k = threadIdx.x; k < bd.nbonds; k += kRowBlock) so[k] = bd.o[k];
-    __syncthreads();
-  }
-  // Workgroup order: with FP64 x each XCD takes a contiguous eighth of the
-  // rows (xcd_block); with FP32 x the dispatch order itself (consecutive
-  // waves on different XCDs) measured faster in back-to-back launches at
-  // D = 8.6e8 (85 vs 89 ms, against 98 vs 102 ms the other way round for
-  // FP64 x).
-  const uint64_t lb = sizeof(XT) == 8 ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-  const uint64_t slot = lb * kRowBlock + threadIdx.x;
-  if (slot >= D) return;
-  const uint64_t i = scheduled_row(sched, slot);
-  uint64_t act[NW];
-  const double diag = row_pass_a<NW, BONDS>(o, bd, reps[i], act);
-  double acc = diag * ld_re(x, i);
-  const uint32_t si = stab[i];
-  const double sr = static_cast<double>(si);
-  const uint32_t *in = entries + woff[lb] * 64 + threadIdx.x;
-  // four terms per step: four x gathers in flight together with the next
-  // step's four entry loads, then the four terms added in template order
-  constexpr int U = 4;
-  int t = 0;
-  int j[U];
-  uint32_t e[U];
-  bool more = any_set<NW>(act);
-#pragma unroll
-  for (int q = 0; q < U; ++q) {
-    j[q] = pop_first<NW>(act);
-    e[q] = j[q] >= 0 ? in[64 * static_cast<uint64_t>(t + q)] : kCacheIndex;
-  }
-  t += U;
-  while (more) {
-    double xv[U];
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-      const uint32_t k = e[q] & kCacheIndex;
-      xv[q] = k != kCacheIndex ? ld_re(x, k) : 0.0;
+  uint32_t t = 0;
+  uint4 group = make_uint4(0, 0, 0, 0);
+  auto store = [&](int64_t k, const OrbitResult &orb, int j) __attribute__((always_inline)) {
+    if (k < 0) return;
+    const int32_t sk = min_only ? static_cast<int32_t>(stab[k]) : orb.count;
+    // from LDS: a load here would wait for every load before it
+    uint32_t cls = CLS ? (units <= 64 * NW ? s_cls[j] : unit_cls[j]) : 0u;
+    if (phases == 2)
+      cls = 2 * cls + (orb.phase != 0 ? 1u : 0u);
+    else if (phases > 2)
+      cls = cls * phases + orb.phase;
+    if (aux) {
+      aux[w0 * 64 + term_pos(t, T, threadIdx.x)] = static_cast<uint16_t>(cls);
+      cls = 0;
     }
-    more = any_set<NW>(act);
-    int jn[U];
-    uint32_t en[U];
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-      jn[q] = pop_first<NW>(act);
-      en[q] = jn[q] >= 0 ? in[64 * static_cast<uint64_t>(t + q)] : kCacheIndex;
+    // a class of 0 keeps the shift (up to 31) harmless
+    const uint32_t ent =
+        static_cast<uint32_t>(k) | (cls << shift) | (sk != si ? 1u << 31 : 0u);
+    // groups of four leave as one 16-byte store: single entries (16 bytes
+    // apart between lanes) made the fill of D = 2.3e8 25 ms longer
+    const uint32_t q = t & 3u;
+    if (t < (T & ~3u)) {
+      group.x = q == 0 ? ent : group.x;
+      group.y = q == 1 ? ent : group.y;
+      group.z = q == 2 ? ent : group.z;
+      group.w = q == 3 ? ent : group.w;
+      if (q == 3u) reinterpret_cast<uint4 *>(out)[64ull * (t >> 2) + threadIdx.x] = group;
+    } else {
+      out[64ull * t + threadIdx.x] = ent;
     }
-    t += U;
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-      const uint32_t k = e[q] & kCacheIndex;
-      if (k == kCacheIndex) continue;
-      double f = 1.0;
-      if (e[q] & kCacheRatio) {
-        const uint32_t ck = stab[k];
-        f = rt.nd ? rt.ratio[rt.div_idx[ck] * rt.nd + rt.div_idx[si]]
-                  : sqrt(static_cast<double>(ck) / sr);
+    ++t;
+  };
+  for (int base = 0; base < units; base += 64 * NW) {
+    uint64_t act[NW];
+    row_active<NW, BONDS>(o, bd, r, base, act);
+    while (any_set<NW>(act)) {
+      const int ja = base + pop_first<NW>(act);
+      int jb = pop_first<NW>(act);
+      jb = jb >= 0 ? base + jb : -1;
+      OrbitResult oa{0, 0, 0, true}, ob{0, 0, 0, false};
+      if (min_only) {
+        oa.rep = orbit_min_generic(ga, r ^ (BONDS ? bd.flip[ja] : o.flip[ja]));
+        if (jb >= 0) {
+          ob.rep = orbit_min_generic(ga, r ^ (BONDS ? bd.flip[jb] : o.flip[jb]));
+          ob.valid = true;
+        }
+      } else {
+        oa = rob.orbit(o, bd, ga, ra, r, ja);
+        if (jb >= 0) ob = rob.orbit(o, bd, ga, ra, r, jb);
       }
-      double c = (BONDS ? so[j[q]] : o.coef_re[j[q]]) * f;
-      c = (e[q] & kCacheNeg) ? -c : c;
-      acc = fma(c, xv[q], acc);
-    }
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-      j[q] = jn[q];
-      e[q] = en[q];
+      int64_t ka, kb;
+      find_index2(ix, oa.rep, oa.valid, ob.rep, ob.valid, ka, kb);
+      store(ka, oa, ja);
+      if (jb >= 0) store(kb, ob, jb);
     }
   }
-  st_re(y, i, acc);
+  if (t < (T & ~3u) && (t & 3u))
+    reinterpret_cast<uint4 *>(out)[64ull * (t >> 2) + threadIdx.x] = group;
+  cnt[slot] = static_cast<uint16_t>(t);
 }
 
-// Row-interleaved block of K vectors from the gather cache: per column the
-// sums of matvec_block_kernel (and so of matvec_real_kernel).
-template <int NW, bool BONDS, int K, class XT, class YT>
+// Vectors that a cached matvec works on: K row-interleaved real vectors, or
+// one complex vector.  Same arithmetic as the matrix-free kernels.
+template <class XT, class YT, int K> struct RealRows {
+  using X = RowK<XT, K>;
+  using Y = RowK<YT, K>;
+  using C = double; // coefficient
+  static constexpr int kGroups = K == 1 ? 2 : 1; // groups of four entries per step
+  static __device__ C pick(double2 c) { return c.x; }
+  double acc[K];
+  __device__ void start(const double *diag, uint64_t slot, bool, const X &x) {
+    const double d = diag[slot];
+#pragma unroll
+    for (int c = 0; c < K; ++c) acc[c] = d * static_cast<double>(x.v[c]);
+  }
+  __device__ void term(C k, double f, const X &x, bool use) {
+    const double cf = k * f;
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      const double t = fma(cf, static_cast<double>(x.v[c]), acc[c]);
+      acc[c] = use ? t : acc[c];
+    }
+  }
+  __device__ Y result() const {
+    Y out;
+#pragma unroll
+    for (int c = 0; c < K; ++c) out.v[c] = static_cast<YT>(acc[c]);
+    return out;
+  }
+};
+
+template <class T> struct ComplexRows { // T = float2 or double2
+  using X = T;
+  using Y = T;
+  using C = double2;
+  static constexpr int kGroups = 2;
+  static __device__ C pick(double2 c) { return c; }
+  double re, im;
+  __device__ void start(const double *diag, uint64_t slot, bool complex_diag, const X &x) {
+    const double dr = complex_diag ? diag[2 * slot] : diag[slot];
+    const double di = complex_diag ? diag[2 * slot + 1] : 0.0;
+    const double xr = static_cast<double>(x.x), xi = static_cast<double>(x.y);
+    re = fma(dr, xr, -(di * xi));
+    im = fma(dr, xi, di * xr);
+  }
+  __device__ void term(C k, double f, const X &x, bool use) {
+    const double kr = k.x * f, ki = k.y * f;
+    const double xr = static_cast<double>(x.x), xi = static_cast<double>(x.y);
+    const double tr = fma(-ki, xi, fma(kr, xr, re));
+    const double ti = fma(ki, xr, fma(kr, xi, im));
+    re = use ? tr : re;
+    im = use ? ti : im;
+  }
+  __device__ Y result() const {
+    Y out;
+    st_c(&out, 0, make_double2(re, im));
+    return out;
+  }
+};
+
+// Matvec from the gather cache: the sums of the matrix-free kernels (same
+// terms, coefficients and order) without orbits or index searches.
+// CM: where a term's coefficient comes from -- 0: one class for all terms
+// (a kernel argument), 1: up to kLdsClasses classes in LDS, 2: the table in
+// memory (read before the gathers of its step: loads complete in order).
+// Bound: the latency of the x gathers, and past the L2 the lines they fetch.
+// One vector takes eight gathers per step (two groups of four entries; D =
+// 6.3e7 ring, FP64: 5.30 ms with four, 5.13 with eight), wider records four
+// (their registers would cost waves).  NT: entries read around the caches,
+// for entry blocks that no cache keeps from one matvec to the next (1.2e9
+// terms: 5.13 -> 4.99 ms; 2e7 terms, 87 MB: 65 -> 80 us, so not there).
+// Against one load per entry, states and bonds read per row and the
+// coefficient by bond, D = 28,968 takes 8.2 us (matrix-free: 72), D = 2.3e8
+// 21.5 ms (24.2).
+constexpr int kLdsClasses = 64;
+constexpr uint64_t kCacheStreamBytes = uint64_t(128) << 20;
+
+template <class R, int CM, bool NT>
 __global__ void __launch_bounds__(kRowBlock)
-    matvec_cached_block_kernel(OpArgs o, BondArgs bd, RatioArgs rt,
-                               const uint64_t *__restrict__ reps, const uint32_t *__restrict__ stab,
-                               uint64_t D, const XT *__restrict__ x, YT *__restrict__ y,
-                               const uint16_t *__restrict__ sched, const uint64_t *__restrict__ woff,
-                               const uint32_t *__restrict__ entries) {
-  __shared__ double so[BONDS ? 64 * NW : 1];
-  if constexpr (BONDS) {
-    for (int k = threadIdx.x; k < bd.nbonds; k += kRowBlock) so[k] = bd.o[k];
+    matvec_cached_kernel(CacheArgs c, RatioArgs rt, const uint32_t *__restrict__ stab, uint64_t D,
+                         const typename R::X *__restrict__ x, typename R::Y *__restrict__ y,
+                         const uint16_t *__restrict__ sched, int contiguous, int complex_diag,
+                         double2 one) {
+  using X = typename R::X;
+  using C = typename R::C;
+  __shared__ C scls[CM == 1 ? kLdsClasses : 1];
+  if constexpr (CM == 1) {
+    if (static_cast<int>(threadIdx.x) < c.nclass)
+      scls[threadIdx.x] =
+          R::pick(make_double2(c.cls[2 * threadIdx.x], c.cls[2 * threadIdx.x + 1]));
     __syncthreads();
   }
-  using Row = RowK<XT, K>;
-  const Row *__restrict__ xr = reinterpret_cast<const Row *>(x);
-  const uint64_t lb = xcd_block(blockIdx.x, gridDim.x);
+  const uint64_t lb = contiguous ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
   const uint64_t slot = lb * kRowBlock + threadIdx.x;
+  const uint64_t w0 = c.woff[lb];
+  const uint32_t T = static_cast<uint32_t>(c.woff[lb + 1] - w0);
   if (slot >= D) return;
+  const uint32_t *in = c.entries + w0 * 64;
+  const uint32_t lane = threadIdx.x;
+  constexpr int Q = R::kGroups;
+  const uint32_t nq = T >> 2;
+  auto group = [&](uint32_t g) {
+    typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+    const v4 *p = reinterpret_cast<const v4 *>(in) + 64ull * g + lane;
+    const v4 none = {0, 0, 0, 0};
+    if constexpr (NT) return g < nq ? __builtin_nontemporal_load(p) : none;
+    return g < nq ? *p : none;
+  };
+  decltype(group(0)) e[Q];
+#pragma unroll
+  for (int z = 0; z < Q; ++z) e[z] = group(z);
   const uint64_t i = scheduled_row(sched, slot);
-  uint64_t act[NW];
-  const double diag = row_pass_a<NW, BONDS>(o, bd, reps[i], act);
-  double acc[K];
-  {
-    const Row xi = xr[i];
-#pragma unroll
-    for (int c = 0; c < K; ++c) acc[c] = diag * static_cast<double>(xi.v[c]);
-  }
-  const uint32_t si = stab[i];
-  const double sr = static_cast<double>(si);
-  const uint32_t *in = entries + woff[lb] * 64 + threadIdx.x;
-  int t = 0;
-  while (any_set<NW>(act)) {
-    const int j = pop_first<NW>(act);
-    const uint32_t e = in[64 * static_cast<uint64_t>(t++)];
-    const uint32_t k = e & kCacheIndex;
-    if (k == kCacheIndex) continue;
-    const Row xk = xr[k];
+  const uint32_t n = c.cnt[slot];
+  R row;
+  row.start(c.diag, slot, complex_diag != 0, x[i]);
+  auto coef = [&](uint32_t ent, uint64_t pos) {
+    if constexpr (CM == 0) return R::pick(one);
+    if constexpr (CM == 1) return scls[(ent >> c.shift) & c.cmask];
+    uint32_t k = c.aux ? c.aux[w0 * 64 + pos] : ((ent >> c.shift) & c.cmask);
+    k = min(k, static_cast<uint32_t>(c.nclass - 1)); // unwritten entries beyond a row's terms
+    return R::pick(make_double2(c.cls[2 * k], c.cls[2 * k + 1]));
+  };
+  auto ratio = [&](uint32_t ent) {
     double f = 1.0;
-    if (e & kCacheRatio) {
-      const uint32_t ck = stab[k];
+    if (ent >> 31) {
+      const uint32_t ck = stab[ent & c.imask], si = stab[i];
       f = rt.nd ? rt.ratio[rt.div_idx[ck] * rt.nd + rt.div_idx[si]]
-                : sqrt(static_cast<double>(ck) / sr);
+                : sqrt(static_cast<double>(ck) / static_cast<double>(si));
     }
-    double cf = (BONDS ? so[j] : o.coef_re[j]) * f;
-    cf = (e & kCacheNeg) ? -cf : cf;
+    return f;
+  };
+  const uint32_t n4 = min(n, nq << 2); // terms in groups
+  for (uint32_t g = 0; g < nq; g += Q) {
+    uint32_t ev[4 * Q];
+    C cv[4 * Q];
+    X xv[4 * Q];
 #pragma unroll
-    for (int c = 0; c < K; ++c) acc[c] = fma(cf, static_cast<double>(xk.v[c]), acc[c]);
+    for (int q = 0; q < 4 * Q; ++q) {
+      ev[q] = e[q / 4][q % 4];
+      cv[q] = coef(ev[q], 256ull * min(g + q / 4, nq - 1) + 4 * lane + q % 4);
+    }
+    // lanes past their row's terms read x[i], which is at hand
+#pragma unroll
+    for (int q = 0; q < 4 * Q; ++q) xv[q] = x[4 * g + q < n4 ? ev[q] & c.imask : i];
+    // after the gathers: loads return in order, and these come from HBM
+#pragma unroll
+    for (int z = 0; z < Q; ++z) e[z] = group(g + Q + z);
+#pragma unroll
+    for (int q = 0; q < 4 * Q; ++q) {
+      const bool use = 4 * g + q < n4;
+      row.term(cv[q], use ? ratio(ev[q]) : 1.0, xv[q], use);
+    }
   }
-  RowK<YT, K> out;
-#pragma unroll
-  for (int c = 0; c < K; ++c) out.v[c] = static_cast<YT>(acc[c]);
-  reinterpret_cast<RowK<YT, K> *>(y)[i] = out;
+  for (uint32_t t = nq << 2; t < T; ++t) {
+    if (t >= n) break;
+    const uint32_t ent = in[64ull * t + lane];
+    row.term(coef(ent, 64ull * t + lane), ratio(ent), x[ent & c.imask], true);
+  }
+  y[i] = row.result();
 }
 
 // Row-interleaved block of K real vectors (x[row * K + c]); per column the
@@ -328,38 +493,86 @@ __global__ void __launch_bounds__(kBlock)
   for (int c = 0; c < K; ++c) y[c * stride + i] = static_cast<B>(yr[i * K + c]);
 }
 
-// Row schedule of one tile (one workgroup per tile): count the active
-// templates of each row (pass A), then a counting sort by count, stable in
-// the row order (thread 0 scatters, so the schedule is deterministic).
-template <int NW, bool BONDS>
-__global__ void __launch_bounds__(kBlock)
+// Row schedule of one tile (one workgroup per tile): the active units of
+// each row, then a counting sort by count, stable in the row order.  Each of
+// the 16 waves owns 256 consecutive rows: a first pass adds up its counts
+// per bin, a scan over (bin, wave) gives its first slot of every bin, a
+// second pass places 64 rows at a time (a row's rank among the lanes of its
+// bin from ballots of the bin's bits).  One serial thread took 205 us for
+// any basis.
+constexpr int kSchedBins = 1024;
+constexpr int kSchedBlock = 1024;
+
+__device__ inline uint64_t same_bin_lanes(uint32_t bin, bool in) {
+  uint64_t m = __ballot(in);
+#pragma unroll
+  for (int b = 0; b < 10; ++b) {
+    const uint64_t v = __ballot((bin >> b) & 1u);
+    m &= ((bin >> b) & 1u) ? v : ~v;
+  }
+  return m;
+}
+
+template <bool BONDS>
+__global__ void __launch_bounds__(kSchedBlock)
     schedule_kernel(OpArgs o, BondArgs bd, const uint64_t *__restrict__ reps, uint64_t D,
                     uint16_t *__restrict__ sched) {
-  constexpr int kBins = 64 * NW + 1;
+  constexpr int kWaves = kSchedBlock / 64, kPerWave = kScheduleTile / kWaves;
   __shared__ uint16_t count_of[kScheduleTile];
-  __shared__ uint32_t offs[kBins];
+  __shared__ uint16_t first[kWaves][kSchedBins]; // at most kScheduleTile rows
+  __shared__ uint32_t part[kSchedBlock];
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kScheduleTile;
   const int rows = static_cast<int>(D - base < kScheduleTile ? D - base : kScheduleTile);
-  for (int t = threadIdx.x; t < kBins; t += kBlock) offs[t] = 0;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  for (int t = threadIdx.x; t < kWaves * kSchedBins; t += kSchedBlock) first[t / kSchedBins][t % kSchedBins] = 0;
   __syncthreads();
-  for (int k = threadIdx.x; k < rows; k += kBlock) {
-    uint64_t act[NW];
-    (void)row_pass_a<NW, BONDS>(o, bd, reps[base + k], act);
-    int c = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) c += __popcll(act[w]);
+  const uint64_t below = (1ull << lane) - 1;
+  for (int k0 = 0; k0 < kPerWave; k0 += 64) {
+    const int k = wid * kPerWave + k0 + lane;
+    const bool in = k < rows;
+    uint32_t c = 0;
+    if (in) c = min(row_count<BONDS>(o, bd, reps[base + k]), static_cast<uint32_t>(kSchedBins - 1));
     count_of[k] = static_cast<uint16_t>(c);
-    atomicAdd(&offs[c], 1u);
+    const uint64_t m = same_bin_lanes(c, in);
+    if (in && (m & below) == 0) first[wid][c] += static_cast<uint16_t>(__popcll(m));
+    __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t run = 0;
-    for (int c = 0; c < kBins; ++c) {
-      const uint32_t h = offs[c];
-      offs[c] = run;
+  // exclusive scan over bins (each thread kSchedBins / kSchedBlock of them), the
+  // waves of a bin in order
+  constexpr int kPer = kSchedBins / kSchedBlock;
+  uint32_t sum = 0;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    for (int w = 0; w < kWaves; ++w) sum += first[w][threadIdx.x * kPer + q];
+  part[threadIdx.x] = sum;
+  __syncthreads();
+  for (int off = 1; off < kSchedBlock; off <<= 1) {
+    const uint32_t v = threadIdx.x >= static_cast<unsigned>(off) ? part[threadIdx.x - off] : 0;
+    __syncthreads();
+    part[threadIdx.x] += v;
+    __syncthreads();
+  }
+  uint32_t run = part[threadIdx.x] - sum;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    for (int w = 0; w < kWaves; ++w) {
+      const uint32_t h = first[w][threadIdx.x * kPer + q];
+      first[w][threadIdx.x * kPer + q] = static_cast<uint16_t>(run);
       run += h;
     }
-    for (int k = 0; k < rows; ++k) sched[base + offs[count_of[k]]++] = static_cast<uint16_t>(k);
+  __syncthreads();
+  for (int k0 = 0; k0 < kPerWave; k0 += 64) {
+    const int k = wid * kPerWave + k0 + lane;
+    const bool in = k < rows;
+    const uint32_t c = count_of[k];
+    const uint64_t m = same_bin_lanes(c, in);
+    const uint32_t at = first[wid][c] + static_cast<uint32_t>(__popcll(m & below));
+    // every lane has read its bin before the bin's first lane moves it on
+    __builtin_amdgcn_wave_barrier();
+    if (in) sched[base + at] = static_cast<uint16_t>(k);
+    if (in && (m & below) == 0) first[wid][c] = static_cast<uint16_t>(at + __popcll(m));
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -593,113 +806,250 @@ template <int METHOD> void dispatch(const MatvecCall &m, const Ctx &c) {
     throw Error(LS_INVALID_DATATYPE, "unsupported matvec type combination");
 }
 
-// Calls f(integral_constant<NW>, bool_constant<BONDS>) for the row-gather
-// kernels' word count; false when the operator has too many templates.
-template <class F> bool with_nw(const Ctx &c, F &&f) {
-  const int units = c.bonds ? c.bd.nbonds : c.o.ntemplates;
-  if (c.bonds && units <= 64)
-    f(std::integral_constant<int, 1>{}, std::true_type{});
-  else if (c.bonds && units <= 128)
-    f(std::integral_constant<int, 2>{}, std::true_type{});
-  else if (!c.bonds && units <= 64)
-    f(std::integral_constant<int, 1>{}, std::false_type{});
-  else if (!c.bonds && units <= 128)
-    f(std::integral_constant<int, 2>{}, std::false_type{});
-  else if (!c.bonds && units <= 256)
-    f(std::integral_constant<int, 4>{}, std::false_type{});
-  else
-    return false;
+// Free memory that an automatically built gather cache leaves untouched.
+constexpr uint64_t kCacheReserve = uint64_t(4) << 30;
+// An automatic cache is built at the first matvec of a basis of kCacheMinRows
+// rows, or when the matrix-free matvec takes about kCacheFirstWork orbit
+// steps (some 300 us) -- the build, one pass over the orbits, then costs
+// about what that matvec would.  Smaller operators build it at their second
+// matvec (a single application is cheaper without), those of up to
+// kCacheTinyRows rows never (the dense solver's unit vectors).
+constexpr uint64_t kCacheMinRows = uint64_t(1) << 20;
+constexpr uint64_t kCacheTinyRows = 64;
+constexpr double kCacheFirstWork = 2e9;
+constexpr uint64_t kCacheMaxClasses = 65536; // 16-bit class numbers
+
+int unit_count(const OperatorTables &t) {
+  return t.bonds ? static_cast<int>(t.h_bond_sites.size()) : t.ntemplates;
+}
+
+// Coefficient classes: every distinct unit coefficient times every phase
+// that an orbit can return, with the products of matvec_complex_kernel (and,
+// for real characters, the sign flip of the real kernels).  False when there
+// are too many.
+bool cache_classes(const Operator &op, GatherCache &gc, hipStream_t s) {
+  const auto &t = op.tables;
+  const auto &bt = op.basis->tables;
+  const int units = unit_count(t);
+  std::vector<uint16_t> of_unit(std::max(units, 1), 0);
+  std::vector<std::pair<double, double>> coefs;
+  std::map<std::pair<uint64_t, uint64_t>, uint16_t> seen;
+  for (int j = 0; j < units; ++j) {
+    const double re = t.bonds ? t.h_bond_o[j] : t.h_coef_re[j];
+    const double im = t.bonds ? 0.0 : t.h_coef_im[j];
+    uint64_t a, b;
+    std::memcpy(&a, &re, 8);
+    std::memcpy(&b, &im, 8);
+    const auto it = seen.emplace(std::make_pair(a, b), static_cast<uint16_t>(coefs.size()));
+    if (it.second) coefs.push_back({re, im});
+    if (coefs.size() > kCacheMaxClasses) return false;
+    of_unit[j] = it.first->second;
+  }
+  if (coefs.empty()) coefs.push_back({0.0, 0.0});
+  const int64_t np = bt.trivial_chars ? 1 : bt.real_chars ? 2 : bt.L;
+  if (static_cast<uint64_t>(np) * coefs.size() > kCacheMaxClasses) return false;
+  std::vector<double> cls;
+  for (const auto &c : coefs)
+    for (int64_t p = 0; p < np; ++p) {
+      double cre = 1.0, cim = 0.0;
+      if (np == 2)
+        cre = p ? -1.0 : 1.0;
+      else
+        phase_values(p, np > 2 ? np : 1, cre, cim);
+      if (t.is_real) {
+        cls.push_back(p ? -c.first : c.first);
+        cls.push_back(0.0);
+      } else {
+        cls.push_back(std::fma(c.first, cre, -(c.second * cim)));
+        cls.push_back(std::fma(c.first, cim, c.second * cre));
+      }
+    }
+  gc.phases = static_cast<int32_t>(np);
+  gc.nclass = static_cast<int32_t>(cls.size() / 2);
+  gc.one[0] = cls[0];
+  gc.one[1] = cls[1];
+  gc.cls.allocate(cls.size());
+  SPINED_HIP(hipMemcpyAsync(gc.cls.ptr, cls.data(), 8 * cls.size(), hipMemcpyHostToDevice, s));
+  gc.unit_cls.allocate(of_unit.size());
+  SPINED_HIP(hipMemcpyAsync(gc.unit_cls.ptr, of_unit.data(), 2 * of_unit.size(),
+                            hipMemcpyHostToDevice, s));
+  SPINED_HIP(hipStreamSynchronize(s)); // the host vectors end here
+  // entry: index bits, class bits, ratio bit
+  int ib = 0, cb = 0;
+  while ((1ull << ib) < op.basis->D) ++ib;
+  while ((1ll << cb) < gc.nclass) ++cb;
+  gc.in_entry = ib + cb <= 31;
+  gc.shift = ib;
+  gc.cmask = gc.in_entry ? static_cast<uint32_t>((1ull << cb) - 1) : 0u;
+  gc.imask = static_cast<uint32_t>((1ull << ib) - 1);
   return true;
 }
 
-// Free memory that an automatically built gather cache leaves untouched,
-// and the smallest basis worth one (the build costs about one matvec).
-constexpr uint64_t kCacheReserve = uint64_t(4) << 30;
-constexpr uint64_t kCacheMinRows = uint64_t(1) << 20;
+template <int METHOD, class F> void with_fill(const Ctx &c, F &&f) {
+  const int units = c.bonds ? c.bd.nbonds : c.o.ntemplates;
+  if (c.bonds && units <= 64)
+    f(std::integral_constant<int, 1>{}, std::true_type{});
+  else if (c.bonds)
+    f(std::integral_constant<int, 2>{}, std::true_type{});
+  else if (units <= 64)
+    f(std::integral_constant<int, 1>{}, std::false_type{});
+  else if (units <= 128)
+    f(std::integral_constant<int, 2>{}, std::false_type{});
+  else
+    f(std::integral_constant<int, 4>{}, std::false_type{});
+}
 
 // Builds the gather cache when it is requested (1), or when it is automatic
-// (-1) and fits in free memory with kCacheReserve to spare.  Caller holds
-// gc.mu.  True when the cache is ready.
+// (-1), due (see kCacheMinRows; repeated: more matvecs are known to follow)
+// and fits in free memory with kCacheReserve to spare.  Caller holds gc.mu.
+// True when the cache is ready.
 template <int METHOD>
 bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t s,
-                  uint64_t reserve = kCacheReserve, uint64_t reusable = 0) {
+                  bool repeated = false, uint64_t reserve = kCacheReserve, uint64_t reusable = 0) {
   if (gc.built) return true;
   const Basis &b = *op.basis;
-  if (gc.request == 0 || !op.tables.is_real || b.D >= kCacheIndex) return false;
+  const int units = unit_count(op.tables);
+  if (gc.request == 0 || b.D > (1ull << 31) || units > 65535) return false;
   struct Building {
     std::atomic<bool> &f;
     explicit Building(std::atomic<bool> &x) : f(x) { f.store(true); }
     ~Building() { f.store(false); }
   } building(gc.building);
-  if (gc.request < 0 && b.D < kCacheMinRows) return false;
+  if (gc.request < 0 && b.D < kCacheMinRows) {
+    if (b.D <= kCacheTinyRows) return false;
+    const double orbit = METHOD == 1 ? 64.0 : 2.0 * b.tables.orbit_cost;
+    if (!repeated && static_cast<double>(b.D) * units * orbit < kCacheFirstWork && gc.calls++ == 0)
+      return false;
+  }
   const uint64_t waves = (b.D + kRowBlock - 1) / kRowBlock;
   const unsigned g = static_cast<unsigned>(waves);
   if (!gc.counted) {
-    DeviceBuffer<uint32_t> wt(waves);
-    DeviceBuffer<uint64_t> tot(1);
-    if (!with_nw(c, [&](auto nw, auto bonds) {
-          cache_count_kernel<decltype(nw)::value, decltype(bonds)::value>
-              <<<g, kRowBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, c.sched, wt.ptr);
-        }))
+    if (!cache_classes(op, gc, s)) {
+      if (gc.request > 0)
+        throw Error(LS_NOT_IMPLEMENTED, "gather cache: too many distinct coefficients");
       return false;
+    }
+    DeviceBuffer<uint32_t> wt(waves);
+    if (c.bonds)
+      cache_count_kernel<true><<<g, kRowBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, c.sched, wt.ptr);
+    else
+      cache_count_kernel<false><<<g, kRowBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, c.sched,
+                                                        wt.ptr);
     SPINED_CHECK_LAUNCH();
-    gc.woff.allocate(waves);
-    scan_counts(wt.ptr, waves, gc.woff.ptr, tot.ptr, s);
+    gc.woff.allocate(waves + 1);
+    scan_counts(wt.ptr, waves, gc.woff.ptr, gc.woff.ptr + waves, s);
     uint64_t t = 0;
-    SPINED_HIP(hipMemcpyAsync(&t, tot.ptr, 8, hipMemcpyDeviceToHost, s));
+    SPINED_HIP(hipMemcpyAsync(&t, gc.woff.ptr + waves, 8, hipMemcpyDeviceToHost, s));
     SPINED_HIP(hipStreamSynchronize(s));
     gc.total = t * kRowBlock;
     gc.counted = true;
   }
+  const uint64_t per_diag = op.tables.is_real ? 1 : 2;
+  const uint64_t n_entries = std::max<uint64_t>(gc.total, 1);
   if (gc.request < 0) {
     size_t free_b = 0, total_b = 0;
     SPINED_HIP(hipMemGetInfo(&free_b, &total_b));
-    free_b += pool_bytes(gc.total * 4) > 0 ? gc.total * 4 : 0; // a pooled block of this size
-    if (free_b < gc.total * 4 + kCacheReserve || free_b + reusable < gc.total * 4 + reserve)
-      return false;
+    const uint64_t blocks[3] = {n_entries * 4, gc.in_entry ? 0 : n_entries * 2, b.D * 8 * per_diag};
+    uint64_t need = b.D * 2;
+    for (uint64_t bytes : blocks) {
+      need += bytes;
+      if (bytes && pool_bytes(bytes) > 0) free_b += bytes; // a pooled block of this size
+    }
+    if (free_b < need + kCacheReserve || free_b + reusable < need + reserve) return false;
   }
   try {
-    // pooled: a rebuild of the same operator's cache takes the block back
+    // pooled: a rebuild of the same operator's cache takes the blocks back
     // without a free and a fresh multi-GB mapping
-    gc.entries.allocate_pooled(std::max<uint64_t>(gc.total, 1));
+    gc.entries.allocate_pooled(n_entries);
+    if (!gc.in_entry) gc.aux.allocate_pooled(n_entries);
+    gc.diag.allocate_pooled(b.D * per_diag);
+    gc.cnt.allocate(b.D);
   } catch (const Error &) {
+    gc.release_entries();
     if (gc.request > 0) throw;
     return false;
   }
-  with_nw(c, [&](auto nw, auto bonds) {
-    cache_fill_kernel<METHOD, decltype(nw)::value, decltype(bonds)::value><<<g, kRowBlock, 0, s>>>(
-        c.o, c.bd, c.ga, c.ra, c.ix, c.stab, c.D, c.sched, gc.woff.ptr, gc.entries.ptr);
+  with_fill<METHOD>(c, [&](auto nw, auto bonds) {
+    auto fill = [&](auto many) {
+      cache_fill_kernel<METHOD, decltype(nw)::value, decltype(bonds)::value, decltype(many)::value>
+          <<<g, kRowBlock, 0, s>>>(c.o, c.bd, c.ga, c.ra, c.ix, c.stab, c.D, c.sched, gc.woff.ptr,
+                                   gc.unit_cls.ptr, gc.phases, gc.shift,
+                                   op.tables.is_real ? 0 : 1, gc.entries.ptr,
+                                   gc.in_entry ? nullptr : gc.aux.ptr, gc.diag.ptr, gc.cnt.ptr);
+    };
+    if (gc.nclass > gc.phases)
+      fill(std::true_type{});
+    else
+      fill(std::false_type{});
   });
   SPINED_CHECK_LAUNCH();
   gc.built = true;
   return true;
 }
 
-template <class XT, class YT>
-void launch_cached(const Ctx &c, const GatherCache &gc, const XT *x, YT *y, hipStream_t s) {
+template <class R>
+void launch_cached(const Operator &op, const Ctx &c, const GatherCache &gc, const void *x, void *y,
+                   bool contiguous, hipStream_t s) {
   const unsigned g = static_cast<unsigned>((c.D + kRowBlock - 1) / kRowBlock);
-  with_nw(c, [&](auto nw, auto bonds) {
-    matvec_cached_kernel<decltype(nw)::value, decltype(bonds)::value, XT, YT>
-        <<<g, kRowBlock, 0, s>>>(c.o, c.bd, c.rt, c.ix.reps, c.stab, c.D, x, y, c.sched,
-                                 gc.woff.ptr, gc.entries.ptr);
-  });
+  const CacheArgs ca{gc.woff.ptr, gc.entries.ptr, gc.in_entry ? nullptr : gc.aux.ptr, gc.diag.ptr,
+                     gc.cnt.ptr,  gc.cls.ptr,     gc.nclass, gc.shift, gc.imask, gc.cmask};
+  const auto *xp = static_cast<const typename R::X *>(x);
+  auto *yp = static_cast<typename R::Y *>(y);
+  const double2 one = make_double2(gc.one[0], gc.one[1]);
+  const int cdiag = op.tables.is_real ? 0 : 1;
+  const bool stream_entries = gc.total * 4 > kCacheStreamBytes;
+  auto go = [&](auto cm) {
+    if (stream_entries)
+      matvec_cached_kernel<R, decltype(cm)::value, true><<<g, kRowBlock, 0, s>>>(
+          ca, c.rt, c.stab, c.D, xp, yp, c.sched, contiguous ? 1 : 0, cdiag, one);
+    else
+      matvec_cached_kernel<R, decltype(cm)::value, false><<<g, kRowBlock, 0, s>>>(
+          ca, c.rt, c.stab, c.D, xp, yp, c.sched, contiguous ? 1 : 0, cdiag, one);
+  };
+  if (gc.nclass == 1)
+    go(std::integral_constant<int, 0>{});
+  else if (gc.in_entry && gc.nclass <= kLdsClasses)
+    go(std::integral_constant<int, 1>{});
+  else
+    go(std::integral_constant<int, 2>{});
   SPINED_CHECK_LAUNCH();
 }
 
-// Real matvec from the gather cache when there is (or can be) one.
+// Workgroup order of the cached kernels: each XCD a contiguous eighth of the
+// rows (xcd_block), or the dispatch order (consecutive waves on different
+// XCDs).  Ring orbits and plain sectors keep the targets of neighbouring
+// rows together, which an XCD's own L2 serves (D = 6.3e7 ring, FP64: 5.13 ms
+// contiguous, 5.44 in dispatch order; D = 5.2e6 without symmetries, FP32:
+// 123 against 161 us); with FP32 x of a ring the two are equal there and the
+// dispatch order is faster at D = 8.6e8 (85 against 89 ms).  Orbits of other
+// groups scatter them, and the XCDs then share the window's lines in the
+// Infinity Cache (6x6 square lattice, FP64: 4.52 ms in dispatch order, 4.75
+// contiguous; FP32: 3.60 against 3.88).
+bool contiguous_rows(const Operator &op, bool f32) {
+  const auto &t = op.basis->tables;
+  if (t.nperm == 1) return true;
+  return t.ring_available && !f32;
+}
+
+// Matvec from the gather cache when there is (or can be) one.
 template <int METHOD> bool try_cached(const MatvecCall &m, const Ctx &c) {
   GatherCache &gc = *m.op->cache;
   std::lock_guard<std::mutex> lk(gc.mu);
-  if (m.no_alloc ? !gc.built : !ensure_cache<METHOD>(*m.op, c, gc, m.stream)) return false;
   using VT = VecType;
-  if (m.xt == VT::F64 && m.yt == VT::F64)
-    launch_cached(c, gc, static_cast<const double *>(m.x), static_cast<double *>(m.y), m.stream);
+  const bool known = (m.xt == m.yt) || (m.xt == VT::F32 && m.yt == VT::F64);
+  if (!known) return false;
+  if (m.no_alloc ? !gc.built : !ensure_cache<METHOD>(*m.op, c, gc, m.stream)) return false;
+  const bool order = contiguous_rows(*m.op, m.xt == VT::F32);
+  if (m.xt == VT::F64)
+    launch_cached<RealRows<double, double, 1>>(*m.op, c, gc, m.x, m.y, order, m.stream);
   else if (m.xt == VT::F32 && m.yt == VT::F32)
-    launch_cached(c, gc, static_cast<const float *>(m.x), static_cast<float *>(m.y), m.stream);
-  else if (m.xt == VT::F32 && m.yt == VT::F64)
-    launch_cached(c, gc, static_cast<const float *>(m.x), static_cast<double *>(m.y), m.stream);
+    launch_cached<RealRows<float, float, 1>>(*m.op, c, gc, m.x, m.y, order, m.stream);
+  else if (m.xt == VT::F32)
+    launch_cached<RealRows<float, double, 1>>(*m.op, c, gc, m.x, m.y, order, m.stream);
+  else if (m.xt == VT::C128)
+    launch_cached<ComplexRows<double2>>(*m.op, c, gc, m.x, m.y, order, m.stream);
   else
-    return false;
+    launch_cached<ComplexRows<float2>>(*m.op, c, gc, m.x, m.y, order, m.stream);
   return true;
 }
 
@@ -738,47 +1088,34 @@ void launch_block(const Ctx &c, int K, const XT *x, YT *y, hipStream_t s) {
   }
 }
 
-template <int K, class XT, class YT>
-void launch_cached_block(const Ctx &c, const GatherCache &gc, const XT *x, YT *y, hipStream_t s) {
-  const unsigned g = static_cast<unsigned>((c.D + kRowBlock - 1) / kRowBlock);
-  with_nw(c, [&](auto nw, auto bonds) {
-    matvec_cached_block_kernel<decltype(nw)::value, decltype(bonds)::value, K, XT, YT>
-        <<<g, kRowBlock, 0, s>>>(c.o, c.bd, c.rt, c.ix.reps, c.stab, c.D, x, y, c.sched,
-                                 gc.woff.ptr, gc.entries.ptr);
-  });
-  SPINED_CHECK_LAUNCH();
-}
-
 template <class XT, class YT>
-void launch_cached_block_k(const Ctx &c, const GatherCache &gc, int K, const XT *x, YT *y,
-                           hipStream_t s) {
-  if (K == 8)
-    launch_cached_block<8>(c, gc, x, y, s);
-  else if (K == 4)
-    launch_cached_block<4>(c, gc, x, y, s);
-  else if (K == 2)
-    launch_cached_block<2>(c, gc, x, y, s);
+void launch_cached_rows(const MatvecBlockCall &m, const Ctx &c, const GatherCache &gc) {
+  const bool order = contiguous_rows(*m.op, false);
+  if (m.K == 8)
+    launch_cached<RealRows<XT, YT, 8>>(*m.op, c, gc, m.x, m.y, order, m.stream);
+  else if (m.K == 4)
+    launch_cached<RealRows<XT, YT, 4>>(*m.op, c, gc, m.x, m.y, order, m.stream);
+  else if (m.K == 2)
+    launch_cached<RealRows<XT, YT, 2>>(*m.op, c, gc, m.x, m.y, order, m.stream);
   else
-    launch_cached_block<1>(c, gc, x, y, s);
+    launch_cached<RealRows<XT, YT, 1>>(*m.op, c, gc, m.x, m.y, order, m.stream);
 }
 
 // Block matvec from the gather cache when there is (or can be) one.
 template <int METHOD> bool try_cached_block(const MatvecBlockCall &m, const Ctx &c) {
   GatherCache &gc = *m.op->cache;
   std::lock_guard<std::mutex> lk(gc.mu);
-  if (!ensure_cache<METHOD>(*m.op, c, gc, m.stream)) return false;
   using VT = VecType;
-  if (m.xt == VT::F64 && m.yt == VT::F64)
-    launch_cached_block_k(c, gc, m.K, static_cast<const double *>(m.x), static_cast<double *>(m.y),
-                          m.stream);
-  else if (m.xt == VT::F32 && m.yt == VT::F32)
-    launch_cached_block_k(c, gc, m.K, static_cast<const float *>(m.x), static_cast<float *>(m.y),
-                          m.stream);
-  else if (m.xt == VT::F32 && m.yt == VT::F64)
-    launch_cached_block_k(c, gc, m.K, static_cast<const float *>(m.x), static_cast<double *>(m.y),
-                          m.stream);
+  const bool f64 = m.xt == VT::F64 && m.yt == VT::F64;
+  const bool f32 = m.xt == VT::F32 && (m.yt == VT::F32 || m.yt == VT::F64);
+  if (!f64 && !f32) return false;
+  if (!ensure_cache<METHOD>(*m.op, c, gc, m.stream)) return false;
+  if (f64)
+    launch_cached_rows<double, double>(m, c, gc);
+  else if (m.yt == VT::F32)
+    launch_cached_rows<float, float>(m, c, gc);
   else
-    return false;
+    launch_cached_rows<float, double>(m, c, gc);
   return true;
 }
 
@@ -860,10 +1197,8 @@ void launch_matvec(const MatvecCall &m) {
     ps = pt.sin_t.ptr;
   }
   const Ctx c = make_ctx(op, pc, ps);
-  if (!cplx) {
-    const bool done = op.orbit_method() == 1 ? try_cached<1>(m, c) : try_cached<0>(m, c);
-    if (done) return;
-  }
+  const bool done = op.orbit_method() == 1 ? try_cached<1>(m, c) : try_cached<0>(m, c);
+  if (done) return;
   if (op.orbit_method() == 1)
     dispatch<1>(m, c);
   else
@@ -876,21 +1211,18 @@ std::vector<Operator *> g_ops; // live operators (their gather caches can be rec
 } // namespace
 
 bool prepare_gather_cache(Operator &op, uint64_t reserve, uint64_t block_bytes) {
-  if (!op.tables.is_real || op.basis->D == 0) return false;
+  if (op.basis->D == 0) return false;
   const Ctx c = make_ctx(op, nullptr, nullptr);
   GatherCache &gc = *op.cache;
   std::lock_guard<std::mutex> lk(gc.mu);
   const uint64_t reusable = pool_bytes(block_bytes);
-  return op.orbit_method() == 1 ? ensure_cache<1>(op, c, gc, stream(), reserve, reusable)
-                                : ensure_cache<0>(op, c, gc, stream(), reserve, reusable);
+  return op.orbit_method() == 1 ? ensure_cache<1>(op, c, gc, stream(), true, reserve, reusable)
+                                : ensure_cache<0>(op, c, gc, stream(), true, reserve, reusable);
 }
 
 void drop_gather_cache_if_built(Operator &op) {
   std::lock_guard<std::mutex> lk(op.cache->mu);
-  if (op.cache->built) {
-    op.cache->built = false;
-    op.cache->entries.release();
-  }
+  if (op.cache->built) op.cache->release_entries();
 }
 
 Operator::Operator() {
@@ -915,10 +1247,7 @@ void reclaim_gather_caches(int device) {
     if (!op->basis || op->basis->device != device) continue;
     GatherCache &gc = *op->cache;
     if (gc.building.load() || !gc.mu.try_lock()) continue;
-    if (gc.built) {
-      gc.built = false;
-      gc.entries.release();
-    }
+    if (gc.built) gc.release_entries();
     gc.mu.unlock();
   }
 }
@@ -979,12 +1308,10 @@ int block_chunk(uint64_t remaining) { return remaining >= 8 ? 8 : remaining >= 4
 void ensure_schedule(Operator &op) {
   std::lock_guard<std::mutex> lk(op.mu);
   const Basis &b = *op.basis;
-  const auto &t = op.tables;
-  const int units = t.bonds ? static_cast<int>(t.h_bond_sites.size()) : t.ntemplates;
-  // automatic: bases of at least one tile with the real row-gather kernels
+  // automatic: bases of at least one tile
   const bool want = op.schedule_request == 1 ||
                     (op.schedule_request < 0 && b.D >= static_cast<uint64_t>(kScheduleTile));
-  if (!want || !t.is_real || units > (t.bonds ? 128 : 256) || b.D == 0) {
+  if (!want || b.D == 0) {
     if (op.schedule_built || op.sched.ptr) drop_gather_cache(op); // cache entries follow the slots
     op.schedule_built = false;
     op.sched.release();
@@ -996,16 +1323,10 @@ void ensure_schedule(Operator &op) {
   op.sched.allocate(b.D);
   const Ctx c = make_ctx(op, nullptr, nullptr);
   const unsigned tiles = static_cast<unsigned>((b.D + kScheduleTile - 1) / kScheduleTile);
-  if (c.bonds && units <= 64)
-    schedule_kernel<1, true><<<tiles, kBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
-  else if (c.bonds)
-    schedule_kernel<2, true><<<tiles, kBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
-  else if (units <= 64)
-    schedule_kernel<1, false><<<tiles, kBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
-  else if (units <= 128)
-    schedule_kernel<2, false><<<tiles, kBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
+  if (c.bonds)
+    schedule_kernel<true><<<tiles, kSchedBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
   else
-    schedule_kernel<4, false><<<tiles, kBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
+    schedule_kernel<false><<<tiles, kSchedBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
   SPINED_CHECK_LAUNCH();
   SPINED_HIP(hipStreamSynchronize(s));
   op.schedule_built = true;

@@ -513,8 +513,12 @@ __host__ __device__ inline bool hop_tops_pair(const RunInfo &ri0, const RunInfo 
   const int bP = aQ == 1 ? ctz64(~(w >> 1)) : 0;
   const uint64_t yq = w << (65 - n);
   const int bQ = aP == 1 ? (yq ? __builtin_clzll(yq) : n) : 0;
-  const RunInfo &riP = ri ? ri1 : ri0;
-  const RunInfo &riQ = ri ? ri0 : ri1;
+  // selected by value: a reference to one of two objects would put both in
+  // scratch memory
+  const RunInfo riP{ri ? ri1.EL : ri0.EL, ri ? ri1.EL1 : ri0.EL1, ri ? ri1.L : ri0.L,
+                    ri ? ri1.usable : ri0.usable};
+  const RunInfo riQ{ri ? ri0.EL : ri1.EL, ri ? ri0.EL1 : ri1.EL1, ri ? ri0.L : ri1.L,
+                    ri ? ri0.usable : ri1.usable};
   const bool okP = riP.usable && aP + bP < n - 1;
   const bool okQ = riQ.usable && aQ + bQ < n - 1;
   int tR2 = j + bP;

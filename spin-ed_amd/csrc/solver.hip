@@ -1170,12 +1170,12 @@ int eigsh(Operator &op, int dtype, uint64_t k, double tol, const spined_eigsh_op
     return LS_SUCCESS;
   }
 
-  // Gather cache (real one-vector solves): a cached matvec costs about a
+  // Gather cache (one-vector solves): a cached matvec costs about a
   // third of the orbit-and-index one, so with an automatic basis size the
   // cache is kept at the price of a smaller Krylov basis, down to
   // kCacheMinBasis vectors; otherwise it gives its memory to the vectors.
-  if (!cplx && block_width(opts.max_block_size) == 1) {
-    const uint64_t blk = n * 8;
+  if (cplx || block_width(opts.max_block_size) == 1) {
+    const uint64_t blk = ne * 8;
     const int extra = 5; // w, start, y, hy and one block of slack
     const int mmin = opts.max_basis_size > 0 ? m : std::min(m, kCacheMinBasis);
     if (prepare_gather_cache(op, static_cast<uint64_t>(mmin + 1 + extra) * blk, blk)) {
