@@ -201,7 +201,8 @@ int spined_operator_get_rows_per_wave(const ls_operator *op);
  * identical.
  * mode: -1 automatic (built when free device memory exceeds it by 4 GiB: at
  * the first matvec of a basis of at least 2^20 rows or of an operator whose
- * matrix-free matvec is long, at the second matvec or at a solve otherwise;
+ * matrix-free matvec is long, at the second call or at a solve otherwise;
+ * not where the states split into halves that need no entries;
  * given back whenever a device allocation of the library needs the memory),
  * 0 off, 1 on (built at the next matvec; an error if it does not fit).  get:
  * 1 while a cache is built.  Changing the row schedule drops the cache. */

@@ -188,6 +188,7 @@ Operator &prepare_operator(const ls_operator *op) {
   ensure_basis_device(b);
   ensure_device(o.tables);
   ensure_schedule(o);
+  ++o.cache->calls;
   return o;
 }
 

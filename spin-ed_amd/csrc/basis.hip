@@ -330,8 +330,46 @@ static void build_rank_index(Basis &b, int mode, hipStream_t s) {
   SPINED_HIP(hipStreamSynchronize(s));
 }
 
+void build_split(const Basis &b, SplitPlan &p, int l) {
+  hipStream_t s = stream();
+  const int nh = b.n - l;
+  // with the flip the top site is down in every row
+  p.nhi = 1u << (b.tables.has_flip ? nh - 1 : nh);
+  std::vector<uint32_t> goff(static_cast<size_t>(p.nhi) + 1), lowoff(l + 2, 0);
+  uint32_t run = 0;
+  // LDS rows: ranks of inactive moves belong to other weights
+  p.largest = static_cast<uint32_t>(binomial(l, l / 2));
+  for (uint32_t hi = 0; hi < p.nhi; ++hi) {
+    goff[hi] = run;
+    const uint64_t c = binomial(l, b.w - __builtin_popcount(hi));
+    run += static_cast<uint32_t>(c);
+  }
+  goff[p.nhi] = run;
+  if (run != b.D) throw Error(LS_INTERNAL_ERROR, "split tables do not match the basis");
+  for (int k = 0; k <= l; ++k) lowoff[k + 1] = lowoff[k] + static_cast<uint32_t>(binomial(l, k));
+  std::vector<uint16_t> state(size_t(1) << l), rank(size_t(1) << l);
+  std::vector<uint32_t> next(lowoff.begin(), lowoff.end() - 1);
+  for (uint32_t x = 0; x < (1u << l); ++x) {
+    const int k = __builtin_popcount(x);
+    rank[x] = static_cast<uint16_t>(next[k] - lowoff[k]);
+    state[next[k]++] = static_cast<uint16_t>(x);
+  }
+  p.goff.allocate(goff.size());
+  p.lowoff.allocate(lowoff.size());
+  p.lowstate.allocate(state.size());
+  p.lowrank.allocate(rank.size());
+  SPINED_HIP(hipMemcpyAsync(p.goff.ptr, goff.data(), 4 * goff.size(), hipMemcpyHostToDevice, s));
+  SPINED_HIP(hipMemcpyAsync(p.lowoff.ptr, lowoff.data(), 4 * lowoff.size(), hipMemcpyHostToDevice, s));
+  SPINED_HIP(hipMemcpyAsync(p.lowstate.ptr, state.data(), 2 * state.size(), hipMemcpyHostToDevice, s));
+  SPINED_HIP(hipMemcpyAsync(p.lowrank.ptr, rank.data(), 2 * rank.size(), hipMemcpyHostToDevice, s));
+  SPINED_HIP(hipStreamSynchronize(s)); // the host vectors end here
+  p.l = l;
+}
+
 void build_index(Basis &b) {
   hipStream_t s = stream();
+  b.split.release();
+  b.split_batch.release();
   if (b.D >= 0xffffffffull)
     throw Error(LS_NOT_IMPLEMENTED, "dimensions of 2^32 - 1 or more are not supported");
   const int rmode = rank_index_mode(b);

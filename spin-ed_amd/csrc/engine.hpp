@@ -16,6 +16,7 @@
 #include "../../include/spined.h"
 #include "common.hpp"
 #include "orbit.hpp"
+#include "split.hpp"
 
 namespace spined {
 
@@ -100,6 +101,22 @@ struct HostStates {
   explicit HostStates(uint64_t n) : data(new uint64_t[n > 0 ? n : 1]), size(n) {}
 };
 
+// Tables of the split row gather (split.hpp) for one cut l.
+struct SplitPlan {
+  int l = -1; // -1: not built
+  uint32_t nhi = 0;
+  uint32_t largest = 0; // low states of the commonest weight
+  DeviceBuffer<uint32_t> goff, lowoff;
+  DeviceBuffer<uint16_t> lowstate, lowrank;
+  void release() {
+    l = -1;
+    goff.release();
+    lowoff.release();
+    lowstate.release();
+    lowrank.release();
+  }
+};
+
 struct Basis {
   std::shared_ptr<const Group> group;
   int n = 0, w = -1, z = 0;
@@ -126,6 +143,12 @@ struct Basis {
   uint64_t hmask = 0;
   int rank_mode = 0;                  // IndexArgs::rank_mode
   DeviceBuffer<uint32_t> rank_tab;    // w x 64 binomials (IndexArgs)
+  // cuts of the single and of the batched matvec, built at their first use
+  SplitPlan split, split_batch;
+  SplitArgs split_args(const SplitPlan &p) const {
+    return SplitArgs{p.goff.ptr, p.lowstate.ptr, p.lowrank.ptr, p.lowoff.ptr, p.nhi,
+                     p.l, n, w, tables.has_flip, tables.flip_phase != 0 ? 1 : 0};
+  }
   std::shared_ptr<HostStates> host_reps; // lazily downloaded
   double seconds_build = 0.0;
 
@@ -162,6 +185,8 @@ void adopt_basis(Basis &b, uint64_t n, const uint64_t *reps); // basis.hip (ls_b
 void validate_representatives(const Basis &b, uint64_t n, const uint64_t *reps);
 void build_index(Basis &b);                                   // basis.hip
 int rank_index_mode(const Basis &b);                          // basis.hip
+// Builds p with l low sites (caller holds b.mu; rank_mode 1).
+void build_split(const Basis &b, SplitPlan &p, int l);        // basis.hip
 // level-2 bucket count for about 2^bits buckets (fills dir when given)
 uint64_t level2_size(const Basis &b, int bits, uint2 *dir);   // basis.hip
 
@@ -227,7 +252,8 @@ struct GatherCache {
   // locking mu a second time
   std::atomic<bool> building{false};
   int request = -1;       // -1 automatic (built when it fits in free memory), 0 off, 1 on
-  int calls = 0;          // matvecs before an automatic cache of a small basis
+  std::atomic<int> calls{0}; // uses of the operator so far (an automatic cache of a small
+                             // basis waits for the second)
   bool counted = false;   // classes, woff and total known
   bool built = false;
   uint64_t total = 0;     // entries
@@ -253,7 +279,6 @@ struct GatherCache {
   void drop() {           // caller holds mu
     release_entries();
     counted = false;
-    calls = 0;
     total = 0;
     woff.release();
     cls.release();
@@ -280,6 +305,9 @@ struct Operator {
   int lanes_per_row = 1;
   bool schedule_built = false;
   DeviceBuffer<uint16_t> sched;
+  // diagonal over the leading low bonds (split.hpp), for the cut of
+  // basis->split; built at the first split matvec (under basis->mu)
+  mutable DeviceBuffer<double> split_dlow;
   std::unique_ptr<GatherCache> cache = std::make_unique<GatherCache>();
   Operator();
   ~Operator();

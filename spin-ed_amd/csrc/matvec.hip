@@ -453,6 +453,38 @@ __global__ void __launch_bounds__(kRowBlock)
   y[i] = row.result();
 }
 
+// ---- split row gather (split.hpp) -------------------------------------------
+__global__ void __launch_bounds__(kBlock)
+    split_dlow_kernel(SplitArgs s, BondArgs bd, double *__restrict__ dlow) {
+  const uint32_t e = blockIdx.x * kBlock + threadIdx.x;
+  if (e < (1u << s.l)) dlow[e] = split_dlow(s, bd, s.lowstate[e]);
+}
+
+// One workgroup per group of rows.  Bound: instruction issue (about 250
+// vector instructions per row and wave) and the two LDS reads of each low
+// bond, so a thread takes up to four rows at once, which share the scalar
+// work of a bond.  D = 5.2e6 (26 sites): 85 us (FP64) and 86 us (FP32) with
+// four rows, 150 and 148 with one; from the gather cache 145 and 117.
+template <class XT, class YT>
+__global__ void __launch_bounds__(kBlock)
+    matvec_split_kernel(SplitArgs s, BondArgs bd, const double *__restrict__ dlow,
+                        const XT *__restrict__ x, YT *__restrict__ y) {
+  extern __shared__ char split_lds[];
+  uint16_t *rank = reinterpret_cast<uint16_t *>(split_lds);
+  XT *xs = reinterpret_cast<XT *>(split_lds + (sizeof(uint16_t) << s.l));
+  const uint32_t hi = static_cast<uint32_t>(xcd_block(blockIdx.x, gridDim.x));
+  const uint32_t g0 = s.goff[hi], cnt = s.goff[hi + 1] - g0;
+  if (cnt == 0) return;
+  const uint4 *rk = reinterpret_cast<const uint4 *>(s.lowrank);
+  for (uint32_t t = threadIdx.x; t < (1u << s.l) / 8; t += kBlock)
+    reinterpret_cast<uint4 *>(rank)[t] = rk[t];
+  for (uint32_t t = threadIdx.x; t < cnt; t += kBlock) xs[t] = x[g0 + t];
+  const SplitBonds sb =
+      split_bonds(s, split_bond(bd, static_cast<int>(threadIdx.x & 63)), hi);
+  __syncthreads();
+  split_group<XT, YT, kBlock>(s, sb, hi, dlow, rank, xs, x, y, g0, cnt);
+}
+
 // Row-interleaved block of K real vectors (x[row * K + c]); per column the
 // same sums as matvec_real_kernel.
 template <int METHOD, int NW, bool BONDS, int K, class XT, class YT>
@@ -812,7 +844,7 @@ constexpr uint64_t kCacheReserve = uint64_t(4) << 30;
 // rows, or when the matrix-free matvec takes about kCacheFirstWork orbit
 // steps (some 300 us) -- the build, one pass over the orbits, then costs
 // about what that matvec would.  Smaller operators build it at their second
-// matvec (a single application is cheaper without), those of up to
+// use (a single application is cheaper without), those of up to
 // kCacheTinyRows rows never (the dense solver's unit vectors).
 constexpr uint64_t kCacheMinRows = uint64_t(1) << 20;
 constexpr uint64_t kCacheTinyRows = 64;
@@ -918,7 +950,7 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
   if (gc.request < 0 && b.D < kCacheMinRows) {
     if (b.D <= kCacheTinyRows) return false;
     const double orbit = METHOD == 1 ? 64.0 : 2.0 * b.tables.orbit_cost;
-    if (!repeated && static_cast<double>(b.D) * units * orbit < kCacheFirstWork && gc.calls++ == 0)
+    if (!repeated && static_cast<double>(b.D) * units * orbit < kCacheFirstWork && gc.calls.load() < 2)
       return false;
   }
   const uint64_t waves = (b.D + kRowBlock - 1) / kRowBlock;
@@ -1029,6 +1061,72 @@ bool contiguous_rows(const Operator &op, bool f32) {
   const auto &t = op.basis->tables;
   if (t.nperm == 1) return true;
   return t.ring_available && !f32;
+}
+
+// Low sites of the split row gather for a basis, or -1 where it does not
+// apply.  Rule: at least 2^20 rows and 256 rows per group.  26 sites at half
+// filling (5.2e6 rows, 635 per group): 85 us against 145 from the gather
+// cache, without its memory and its build; 24 sites (1.4e6 rows): 28 against
+// 31; 22 sites (3.5e5): 11.5 against 11.5.  Away from half filling groups
+// shrink: 28 sites, 7 up (72 per group): 210 us against 23.
+constexpr uint64_t kSplitMinRows = uint64_t(1) << 20;
+constexpr uint64_t kSplitMinGroup = 256;
+
+int split_low(const Operator &op) {
+  const Basis &b = *op.basis;
+  const auto &t = op.tables;
+  if (b.index_kind != 2 || b.rank_mode != 1 || !t.bonds || !t.is_real) return -1;
+  if (static_cast<int>(t.h_bond_sites.size()) > kSplitMaxBonds || b.D < kSplitMinRows) return -1;
+  const int l = b.n <= 26 ? 12 : kSplitMaxLow;
+  const int nh = b.n - l - (b.tables.has_flip ? 1 : 0);
+  if (nh < 1 || nh > kSplitMaxHigh || (b.D >> nh) < kSplitMinGroup) return -1;
+  return l;
+}
+
+template <class XT, class YT>
+void launch_split(const Operator &op, const Ctx &c, const XT *x, YT *y, hipStream_t s) {
+  const Basis &b = *op.basis;
+  const SplitPlan &p = b.split;
+  const size_t lds = (sizeof(uint16_t) << p.l) + sizeof(XT) * p.largest;
+  matvec_split_kernel<<<p.nhi, kBlock, lds, s>>>(b.split_args(p), c.bd, op.split_dlow.ptr, x, y);
+  SPINED_CHECK_LAUNCH();
+}
+
+// Real matvec by the split row gather, unless a gather cache is asked for or
+// several lanes per row are.
+bool try_split(const MatvecCall &m, const Ctx &c) {
+  using VT = VecType;
+  const Operator &op = *m.op;
+  if (m.xt == VT::C64 || m.xt == VT::C128 || c.lanes != 1) return false;
+  if (m.xt == VT::F64 && m.yt != VT::F64) return false;
+  const int l = split_low(op);
+  if (l < 0 || op.orbit_method() != 0) return false;
+  {
+    std::lock_guard<std::mutex> lk(op.cache->mu);
+    if (op.cache->request > 0 || op.cache->built) return false;
+  }
+  Basis &b = *op.basis;
+  {
+    std::lock_guard<std::mutex> lk(b.mu);
+    if (b.split.l < 0) {
+      if (m.no_alloc) return false;
+      build_split(b, b.split, l);
+    }
+    if (!op.split_dlow.ptr) {
+      if (m.no_alloc) return false;
+      op.split_dlow.allocate(size_t(1) << l);
+      split_dlow_kernel<<<grid_for(uint64_t(1) << l), kBlock, 0, m.stream>>>(
+          b.split_args(b.split), c.bd, op.split_dlow.ptr);
+      SPINED_CHECK_LAUNCH();
+    }
+  }
+  if (m.xt == VT::F64)
+    launch_split(op, c, static_cast<const double *>(m.x), static_cast<double *>(m.y), m.stream);
+  else if (m.yt == VT::F32)
+    launch_split(op, c, static_cast<const float *>(m.x), static_cast<float *>(m.y), m.stream);
+  else
+    launch_split(op, c, static_cast<const float *>(m.x), static_cast<double *>(m.y), m.stream);
+  return true;
 }
 
 // Matvec from the gather cache when there is (or can be) one.
@@ -1197,6 +1295,7 @@ void launch_matvec(const MatvecCall &m) {
     ps = pt.sin_t.ptr;
   }
   const Ctx c = make_ctx(op, pc, ps);
+  if (try_split(m, c)) return;
   const bool done = op.orbit_method() == 1 ? try_cached<1>(m, c) : try_cached<0>(m, c);
   if (done) return;
   if (op.orbit_method() == 1)
@@ -1215,6 +1314,8 @@ bool prepare_gather_cache(Operator &op, uint64_t reserve, uint64_t block_bytes) 
   const Ctx c = make_ctx(op, nullptr, nullptr);
   GatherCache &gc = *op.cache;
   std::lock_guard<std::mutex> lk(gc.mu);
+  // an automatic cache is not built where the split row gather serves
+  if (gc.request < 0 && !gc.built && c.lanes == 1 && split_low(op) >= 0) return false;
   const uint64_t reusable = pool_bytes(block_bytes);
   return op.orbit_method() == 1 ? ensure_cache<1>(op, c, gc, stream(), true, reserve, reusable)
                                 : ensure_cache<0>(op, c, gc, stream(), true, reserve, reusable);
