@@ -45,6 +45,7 @@
 #include "handles.hpp"
 #include "jacobi.hpp"
 #include "rowgather.hpp"
+#include "split.hpp"
 
 namespace spined {
 
@@ -53,11 +54,17 @@ namespace {
 constexpr int kTile = 256;      // rows per tile = threads per workgroup
 constexpr int kMaxM = 24;       // basis size limit of the batched solver
 constexpr int kPS = kMaxM + 4;  // partial slots per member and reduction
-constexpr int kChunk = 8;       // dots per pass
+constexpr int kChunk = 16;      // dots per pass
 constexpr int kMaxKeep = kMaxM / 2; // kept Ritz vectors (keep = m / 2)
 constexpr int kMaxTeam = 128;     // team capacity (partial slots)
 constexpr int kDefaultTeamCap = 32;
 constexpr uint64_t kRowsPerMember = 32768;
+constexpr uint64_t kMinRowsPerMember = 4096;
+// split row gather (split.hpp): low sites, and the rows per group below
+// which an instance keeps the row-by-row gather
+constexpr int kSplitLowSites = 12;
+constexpr uint64_t kSplitMinGroup = 64;
+constexpr uint32_t kSplitGroup = 924; // largest group: C(12, 6)
 constexpr uint32_t kChunkTiles = 4; // matvec rows handed out per grab: 1024
 constexpr int kBarWords = 3;        // per instance: arrivals, generation, chunk counter
 // s_memrealtime runs at 100 MHz: 60 s
@@ -80,6 +87,9 @@ struct PInst {
   double *out;    // [0] lambda [1] residual [2] cycles [3] matvecs [4] finish ticks [5] status
   uint32_t team;
   uint32_t ntiles;
+  SplitArgs sp;        // split row gather; sp.l == 0: row by row
+  const double *dlow;  // its diagonal sums (2^l)
+  uint32_t groups_per_chunk;
 };
 
 struct Slot {
@@ -185,30 +195,53 @@ __device__ inline double matvec_row(const PInst &I, const IndexArgs &ix, uint64_
 }
 
 // partials of V_q . w for q in [0, nv) and (with ww) w . w in slot nv, over
-// the member's rows, into the member's partial slots
+// the member's rows, into the member's partial slots.  Up to kChunk vectors
+// per pass: with 16 the default basis takes one pass over w, and 17 loads
+// of a row are in flight.
 __device__ void dots_pass(Team &tm, int nv, bool ww) {
   const PInst &I = tm.I;
   double *dst = tm.pm_mine();
-  const int total = nv + (ww ? 1 : 0);
-  for (int q0 = 0; q0 < total; q0 += kChunk) {
-    double acc[kChunk];
+  for (int q0 = 0; q0 < nv; q0 += kChunk) {
+    const int nq = std::min(kChunk, nv - q0);
+    const bool last = q0 + nq == nv;
+    double acc[kChunk + 1];
 #pragma unroll
-    for (int c = 0; c < kChunk; ++c) acc[c] = 0.0;
+    for (int c = 0; c <= kChunk; ++c) acc[c] = 0.0;
+    const double *V0 = I.V + static_cast<uint64_t>(q0) * I.D;
     for (uint32_t tile = tm.k; tile < I.ntiles; tile += tm.t) {
       const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
       if (r >= I.D) continue;
       const double wr = I.w[r];
+      double v[kChunk];
+      // slots past nq read the first vector: every load is unconditional
 #pragma unroll
-      for (int c = 0; c < kChunk; ++c) {
-        const int q = q0 + c;
-        if (q < nv)
-          acc[c] = fma(I.V[static_cast<uint64_t>(q) * I.D + r], wr, acc[c]);
-        else if (q == nv && ww)
-          acc[c] = fma(wr, wr, acc[c]);
-      }
+      for (int c = 0; c < kChunk; ++c) v[c] = V0[(c < nq ? static_cast<uint64_t>(c) : 0) * I.D + r];
+#pragma unroll
+      for (int c = 0; c < kChunk; ++c) acc[c] = c < nq ? fma(v[c], wr, acc[c]) : acc[c];
+      acc[kChunk] = fma(wr, wr, acc[kChunk]);
     }
-    block_sums<kChunk>(acc, std::min(kChunk, total - q0), dst + q0);
+    const int total = nq + (ww && last ? 1 : 0);
+#pragma unroll
+    for (int c = 0; c < kChunk; ++c) acc[c] = c == nq ? acc[kChunk] : acc[c];
+    block_sums<kChunk + 1>(acc, total, dst + q0);
   }
+}
+
+// sum_{q < nv} h[q] V_q[r], in q order, kLoads vectors read at a time (a
+// plain loop keeps one read in flight; 48 rings of 12..24 sites: 142 ms with
+// it)
+constexpr int kLoads = 8;
+__device__ inline double row_sum(const PInst &I, int nv, const double *h, uint64_t r) {
+  double s = 0.0;
+  for (int q0 = 0; q0 < nv; q0 += kLoads) {
+    double v[kLoads];
+#pragma unroll
+    for (int c = 0; c < kLoads; ++c)
+      v[c] = I.V[static_cast<uint64_t>(q0 + c < nv ? q0 + c : q0) * I.D + r];
+#pragma unroll
+    for (int c = 0; c < kLoads; ++c) s = q0 + c < nv ? fma(h[q0 + c], v[c], s) : s;
+  }
+  return s;
 }
 
 // w -= sum_{q < nv} h[q] V_q over the member's rows; then the partials of
@@ -219,9 +252,7 @@ __device__ void update_pass(Team &tm, int nv, const double *h, bool dots) {
   for (uint32_t tile = tm.k; tile < I.ntiles; tile += tm.t) {
     const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
     if (r >= I.D) continue;
-    double s = 0.0;
-    for (int q = 0; q < nv; ++q) s = fma(h[q], I.V[static_cast<uint64_t>(q) * I.D + r], s);
-    const double wr = I.w[r] - s;
+    const double wr = I.w[r] - row_sum(I, nv, h, r);
     I.w[r] = wr;
     acc[0] = fma(wr, wr, acc[0]);
   }
@@ -238,9 +269,7 @@ __device__ void update_store_pass(Team &tm, int nv, const double *h, double inv,
   for (uint32_t tile = tm.k; tile < I.ntiles; tile += tm.t) {
     const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
     if (r >= I.D) continue;
-    double s = 0.0;
-    for (int q = 0; q < nv; ++q) s = fma(h[q], I.V[static_cast<uint64_t>(q) * I.D + r], s);
-    v[r] = (I.w[r] - s) * inv;
+    v[r] = (I.w[r] - row_sum(I, nv, h, r)) * inv;
   }
 }
 
@@ -258,8 +287,20 @@ __device__ void solve_instance(const PInst &I, uint32_t inst_id, uint32_t member
   // binomial table is read from LDS by every lookup
   __shared__ uint32_t sRank[METHOD == 0 ? kRankMaxW * 64 : 1];
   IndexArgs ix = I.ix;
+  // split row gather: the same LDS holds the rank table of the low states,
+  // and each lane keeps its bond
+  static_assert(kRankMaxW * 64 * 4 >= (2 << kSplitLowSites), "rank table fits");
+  __shared__ double sX[METHOD == 0 ? kSplitGroup : 1];
+  const bool split = METHOD == 0 && I.sp.l > 0;
+  SplitBond my_bond{0.0, 0.0, 0.0, 0, false};
+  uint16_t *srank16 = reinterpret_cast<uint16_t *>(sRank);
+  if (split) {
+    my_bond = split_bond(I.bd, static_cast<int>(threadIdx.x & 63));
+    for (int e = threadIdx.x; e < (1 << I.sp.l); e += kTile) srank16[e] = I.sp.lowrank[e];
+    __syncthreads();
+  }
   if constexpr (METHOD == 0) {
-    if (ix.rank_mode == 1) {
+    if (!split && ix.rank_mode == 1) {
       for (int e = threadIdx.x; e < ix.rank_w * 64; e += kTile) sRank[e] = ix.rank_tab[e];
       __syncthreads();
     }
@@ -285,10 +326,37 @@ __device__ void solve_instance(const PInst &I, uint32_t inst_id, uint32_t member
   // before the current chunk runs.  A row's sum does not depend on who
   // computes it.  Ends with a team barrier (the Gram-Schmidt passes read
   // their own rows of w); false on abort.
+  // With the split row gather a chunk is a few groups of rows instead.
   __shared__ uint32_t s_chunk;
   uint32_t mv_round = 0;
-  auto matvec_chunks = [&](const double *x) {
-    const uint32_t nch = (I.ntiles + kChunkTiles - 1) / kChunkTiles;
+  auto chunk_rows = [&](uint32_t g, const double *x, double *out) {
+    if (split) {
+      const uint32_t h_end = std::min((g + 1) * I.groups_per_chunk, I.sp.nhi);
+      for (uint32_t h0 = g * I.groups_per_chunk; h0 < h_end; ++h0) {
+        const uint32_t hi = __builtin_amdgcn_readfirstlane(h0);
+        const uint32_t g0 = I.sp.goff[hi], cnt = I.sp.goff[hi + 1] - g0;
+        if (cnt == 0) continue;
+        const SplitBonds sb = split_bonds(I.sp, my_bond, hi);
+        for (uint32_t t = threadIdx.x; t < cnt; t += kTile) sX[t] = x[g0 + t];
+        __syncthreads();
+        split_group<double, double, kTile>(I.sp, sb, hi, I.dlow, srank16, sX, x, out, g0, cnt);
+        __syncthreads(); // sX is read until here
+      }
+      return;
+    }
+    const uint32_t t_end = std::min((g + 1) * kChunkTiles, I.ntiles);
+    for (uint32_t tile = g * kChunkTiles; tile < t_end; ++tile) {
+      const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
+      if (r < D) out[r] = mv(r, x);
+    }
+  };
+  auto matvec_chunks = [&](const double *x, double *out) {
+    const uint32_t nch = split ? (I.sp.nhi + I.groups_per_chunk - 1) / I.groups_per_chunk
+                               : (I.ntiles + kChunkTiles - 1) / kChunkTiles;
+    if (tm.t == 1) {
+      for (uint32_t g = 0; g < nch; ++g) chunk_rows(g, x, out);
+      return tm.sync();
+    }
     const uint32_t base = mv_round++ * (nch + tm.t);
     unsigned *ctr = I.bar + 2;
     if (threadIdx.x == 0) s_chunk = atomicAdd(ctr, 1u) - base;
@@ -297,11 +365,7 @@ __device__ void solve_instance(const PInst &I, uint32_t inst_id, uint32_t member
     __syncthreads();
     while (g < nch) {
       if (threadIdx.x == 0) s_chunk = atomicAdd(ctr, 1u) - base;
-      const uint32_t t_end = std::min((g + 1) * kChunkTiles, I.ntiles);
-      for (uint32_t tile = g * kChunkTiles; tile < t_end; ++tile) {
-        const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
-        if (r < D) I.w[r] = mv(r, x);
-      }
+      chunk_rows(g, x, out);
       __syncthreads();
       g = s_chunk;
       __syncthreads();
@@ -341,14 +405,7 @@ __device__ void solve_instance(const PInst &I, uint32_t inst_id, uint32_t member
     for (int j = j0; j < mm; ++j) {
       // w = H v_j (own rows); dots with V_0..V_j and w.w
       const double *x = vec(j);
-      if (tm.t > 1) {
-        if (!matvec_chunks(x)) return;
-      } else {
-        for (uint32_t tile = 0; tile < I.ntiles; ++tile) {
-          const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
-          if (r < D) I.w[r] = mv(r, x);
-        }
-      }
+      if (!matvec_chunks(x, I.w)) return;
       ++matvecs;
       dots_pass(tm, j + 1, true);
       if (!tm.reduce(j + 2, sh1)) return;
@@ -408,18 +465,16 @@ __device__ void solve_instance(const PInst &I, uint32_t inst_id, uint32_t member
       for (uint32_t tile = member; tile < I.ntiles; tile += tm.t) {
         const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
         if (r >= D) continue;
-        double acc = 0.0;
-        for (int q = 0; q < msz; ++q) acc = fma(sS[q], vec(q)[r], acc);
-        I.w[r] = acc;
+        I.w[r] = row_sum(I, msz, sS, r);
       }
       if (!tm.sync()) return;
       double *hy = vec(m + 1);
+      if (!matvec_chunks(I.w, hy)) return;
       double acc2[2] = {0.0, 0.0};
       for (uint32_t tile = member; tile < I.ntiles; tile += tm.t) {
         const uint64_t r = static_cast<uint64_t>(tile) * kTile + threadIdx.x;
         if (r >= D) continue;
-        const double h = mv(r, I.w);
-        hy[r] = h;
+        const double h = hy[r];
         const double y = I.w[r];
         acc2[0] = fma(y, h, acc2[0]);
         acc2[1] = fma(y, y, acc2[1]);
@@ -460,10 +515,15 @@ __device__ void solve_instance(const PInst &I, uint32_t inst_id, uint32_t member
       double out[kMaxKeep];
 #pragma unroll
       for (int i = 0; i < kMaxKeep; ++i) out[i] = 0.0;
-      for (int q = 0; q < msz; ++q) {
-        const double x = vec(q)[r];
+      for (int q0 = 0; q0 < msz; q0 += kLoads) {
+        double v[kLoads];
 #pragma unroll
-        for (int i = 0; i < kMaxKeep; ++i) out[i] = fma(sC[q * kMaxKeep + i], x, out[i]);
+        for (int c = 0; c < kLoads; ++c) v[c] = vec(q0 + c < msz ? q0 + c : q0)[r];
+        for (int c = 0; c < kLoads && q0 + c < msz; ++c) {
+#pragma unroll
+          for (int i = 0; i < kMaxKeep; ++i)
+            out[i] = fma(sC[(q0 + c) * kMaxKeep + i], v[c], out[i]);
+        }
       }
       const double last = vec(msz)[r];
 #pragma unroll
@@ -489,7 +549,7 @@ __device__ void solve_instance(const PInst &I, uint32_t inst_id, uint32_t member
 }
 
 template <int METHOD, int NW>
-__global__ void __launch_bounds__(kTile)
+__global__ void __launch_bounds__(kTile, 4)
     batch_persistent_kernel(const PInst *__restrict__ insts, const Slot *__restrict__ slots,
                             uint32_t nslots, unsigned *ticket, int m, int keep, double tol,
                             int max_cycles, uint64_t seed, int *abort, uint64_t *t_start) {
@@ -538,6 +598,17 @@ int resident_blocks() {
 
 } // namespace
 
+namespace {
+__global__ void __launch_bounds__(kTile) batch_dlow_kernel(const PInst *__restrict__ insts,
+                                                           double *__restrict__ dlow) {
+  const PInst &I = insts[blockIdx.y];
+  const uint32_t e = blockIdx.x * kTile + threadIdx.x;
+  if (I.sp.l > 0 && e < (1u << I.sp.l))
+    dlow[(static_cast<uint64_t>(blockIdx.y) << kSplitLowSites) + e] =
+        split_dlow(I.sp, I.bd, I.sp.lowstate[e]);
+}
+} // namespace
+
 // One batched solve; see the file comment.
 int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint64_t seed,
                 int max_cycles, double *evals, double *rnorms, int32_t *cycles_out,
@@ -569,11 +640,12 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
   // them, for tuning)
   uint64_t rows_per_member = kRowsPerMember;
   int team_cap = kDefaultTeamCap;
+  const bool tuned = std::getenv("SPINED_BATCH_ROWS_PER_MEMBER") || std::getenv("SPINED_BATCH_MAX_TEAM");
   if (const char *e = std::getenv("SPINED_BATCH_ROWS_PER_MEMBER"))
     rows_per_member = std::max<uint64_t>(kTile, std::strtoull(e, nullptr, 10));
   if (const char *e = std::getenv("SPINED_BATCH_MAX_TEAM"))
     team_cap = std::max(1, std::min(kMaxTeam, std::atoi(e)));
-  const uint32_t max_team = static_cast<uint32_t>(std::max(1, std::min(team_cap, resident)));
+  uint32_t max_team = static_cast<uint32_t>(std::max(1, std::min(team_cap, resident)));
 
   // per-instance storage
   std::vector<uint64_t> voff(n_inst);
@@ -590,6 +662,7 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
   DeviceBuffer<double> pm(pm_per * n_inst);
   DeviceBuffer<double> outs(8ull * n_inst);
   DeviceBuffer<unsigned> bars(static_cast<uint64_t>(kBarWords) * n_inst);
+  DeviceBuffer<double> dlow(static_cast<uint64_t>(n_inst) << kSplitLowSites);
   std::vector<PInst> hinst(n_inst);
   for (int i = 0; i < n_inst; ++i) {
     Operator &op = *ops[i];
@@ -611,9 +684,46 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
     I.bar = bars.ptr + static_cast<uint64_t>(kBarWords) * i;
     I.out = outs.ptr + 8ull * i;
     I.ntiles = static_cast<uint32_t>((b.D + kTile - 1) / kTile);
-    const uint64_t want = (b.D + rows_per_member - 1) / rows_per_member;
-    I.team = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>({want, max_team, I.ntiles})));
+    I.sp = SplitArgs{};
+    I.dlow = dlow.ptr + (static_cast<uint64_t>(i) << kSplitLowSites);
+    I.groups_per_chunk = 1;
+    // every site above the low ones counts as high; the top one is down in
+    // each row of a flip sector, so it never makes a group of its own
+    const int l = std::min(kSplitLowSites, b.n - 1);
+    const int nh = b.n - l - (b.tables.has_flip ? 1 : 0);
+    if (method == 0 && b.index_kind == 2 && b.rank_mode == 1 && t.keeps_weight &&
+        t.h_bond_sites.size() <= static_cast<size_t>(kSplitMaxBonds) && nh >= 0 &&
+        nh <= kSplitMaxHigh && (b.D >> nh) >= kSplitMinGroup) {
+      std::lock_guard<std::mutex> lk(b.mu);
+      if (b.split_batch.l < 0) build_split(b, b.split_batch, l);
+      I.sp = b.split_args(b.split_batch);
+      I.groups_per_chunk = static_cast<uint32_t>(std::max<uint64_t>(1, (kChunkTiles * kTile) / std::max<uint64_t>(1, b.D >> nh)));
+    }
   }
+  // Team sizes: rows_per_member rows a workgroup, at most max_team of them;
+  // when that leaves workgroups without a slot, half the rows and twice the
+  // team at a time.  Not up to the last workgroup: every team barrier writes
+  // back and invalidates its XCDs' L2 once per member, and with 1,024
+  // members waiting the barriers take longer than the work (8 rings of 24
+  // sites: 122 ms in teams of 32, 121 of 64, 207 of 128; one ring: 82, 45,
+  // 29; 48 rings of 12 .. 24: 146, 124, 177).
+  auto team_of = [&](uint64_t D, uint32_t ntiles, uint64_t rows, uint32_t cap) {
+    const uint64_t want = (D + rows - 1) / rows;
+    return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>({want, cap, ntiles})));
+  };
+  auto slots_for = [&](uint64_t rows, uint32_t cap) {
+    uint64_t n = 0;
+    for (const auto &I : hinst) n += team_of(I.D, I.ntiles, rows, cap);
+    return n;
+  };
+  while (!tuned && rows_per_member > kMinRowsPerMember) {
+    const uint32_t cap = static_cast<uint32_t>(
+        std::min<uint64_t>({2ull * max_team, kMaxTeam, static_cast<uint64_t>(resident)}));
+    if (slots_for(rows_per_member / 2, cap) > static_cast<uint64_t>(resident) * 2 / 3) break;
+    rows_per_member /= 2;
+    max_team = cap;
+  }
+  for (auto &I : hinst) I.team = team_of(I.D, I.ntiles, rows_per_member, max_team);
   // queue: largest instances first (their teams form first), members in order
   std::vector<int> order(n_inst);
   std::iota(order.begin(), order.end(), 0);
@@ -633,6 +743,9 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
   const uint64_t nbar = static_cast<uint64_t>(kBarWords) * n_inst;
   batch_init_kernel<<<static_cast<unsigned>((nbar + 255) / 256), 256, 0, s>>>(
       ticket.ptr, abort_flag.ptr, t_start.ptr, bars.ptr, nbar);
+  SPINED_CHECK_LAUNCH();
+  batch_dlow_kernel<<<dim3((1 << kSplitLowSites) / kTile, static_cast<unsigned>(n_inst)), kTile, 0, s>>>(
+      dinst.ptr, dlow.ptr);
   SPINED_CHECK_LAUNCH();
   // one workgroup per slot at most, no more than fit on the device at once
   const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(nslots, static_cast<uint64_t>(resident)));
