@@ -87,12 +87,9 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// h[i] (+)= sum_b partial[i*G + b], fixed order (deterministic).  Does
-// nothing when skip is given and *skip != 0.
+// h[i] (+)= sum_b partial[i*G + b], fixed order (deterministic).
 __global__ void reduce_partials_kernel(const double *__restrict__ partial, int nvec, int G,
-                                       double *__restrict__ h, int accumulate,
-                                       const int *__restrict__ skip = nullptr) {
-  if (skip && *skip) return;
+                                       double *__restrict__ h, int accumulate) {
   const int i = blockIdx.x;
   __shared__ double lds[kBlock];
   double s = 0.0;
@@ -189,6 +186,24 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 constexpr int kFuseMax = 32; // vectors held in registers by the fused passes
+
+// Sum of G partials by one wave, in the order of reduce_partials_kernel
+// (256 strided sums, then the halving tree); the result in lane 0.
+__device__ inline double wave_partial_sum(const double *__restrict__ p, int G, int lane) {
+  double s[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    s[c] = 0.0;
+    for (int b = lane + 64 * c; b < G; b += kBlock) s[c] += p[b];
+  }
+  double v = (s[0] + s[2]) + (s[1] + s[3]);
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  return v;
+}
+// Invariant subspace: the step's beta against its diagonal entry of T.
+__device__ inline double broke_down(double beta, double tjj) {
+  return beta <= 1e-12 * fmax(1.0, fabs(tjj)) ? 1.0 : 0.0;
+}
 // The second Gram-Schmidt pass runs only when the first update keeps less
 // than this fraction of |w| (second_pass_test_kernel).
 constexpr double kSecondPassEta = 1e-2;
@@ -252,20 +267,34 @@ __global__ void __launch_bounds__(kBlock)
   block_partials<NQ>(acc, nvec, partial);
 }
 
-// Last update fused with the norm: w[r] -= sum_i h2[i] V_i[r]; partial
-// sums of w[r]^2 (the norm_w multidot's arithmetic).  When *skip != 0 (the
-// first pass was the only one) the update uses h1 and stores the next basis
-// vector directly, vnext[r] = (w[r] - sum_i h1[i] V_i[r]) / *beta, with the
-// Pythagorean beta of second_pass_test_kernel (w and the partials are then
-// left alone).
+// Last update fused with the norm.  When *skip != 0 (the first pass was the
+// only one) the update uses h1 and stores the next basis vector directly,
+// vnext[r] = (w[r] - sum_i h1[i] V_i[r]) / *beta, with the Pythagorean beta
+// of first_pass_kernel.  Otherwise every workgroup sums the second pass's
+// partials h2p into h2 (a launch of its own costs more than the sums), then
+// w[r] -= sum_i h2[i] V_i[r], and partial sums of w[r]^2.
 template <class VT, int NQ>
 __global__ void __launch_bounds__(kBlock)
-    sub_norm_kernel(const VT *const *__restrict__ V, int nvec, const double *__restrict__ h2,
-                    double *__restrict__ w, uint64_t n, double *__restrict__ partial,
-                    const double *__restrict__ h1, const int *__restrict__ skip,
-                    VT *__restrict__ vnext, const double *__restrict__ beta) {
+    sub_norm_kernel(const VT *const *__restrict__ V, int nvec, const double *__restrict__ h2p,
+                    double *__restrict__ h2, double *__restrict__ w, uint64_t n,
+                    double *__restrict__ partial, const double *__restrict__ h1,
+                    const int *__restrict__ skip, VT *__restrict__ vnext,
+                    const double *__restrict__ beta) {
   const bool store = *skip != 0;
-  const double *c = store ? h1 : h2;
+  __shared__ double c[NQ];
+  if (store) {
+    if (static_cast<int>(threadIdx.x) < nvec) c[threadIdx.x] = h1[threadIdx.x];
+  } else {
+    for (int i = threadIdx.x >> 6; i < nvec; i += kBlock / 64) {
+      const double v = wave_partial_sum(h2p + static_cast<uint64_t>(i) * gridDim.x, gridDim.x,
+                                        static_cast<int>(threadIdx.x & 63));
+      if ((threadIdx.x & 63) == 0) {
+        c[i] = v;
+        if (blockIdx.x == 0) h2[i] = v;
+      }
+    }
+  }
+  __syncthreads();
   const double b = store ? *beta : 0.0;
   const double inv = b > 0.0 ? 1.0 / b : 0.0;
   const VT *vp[NQ];
@@ -320,37 +349,89 @@ __global__ void __launch_bounds__(kBlock)
   block_partials<NQ + 1>(out, nvec + 1, partial);
 }
 
-// Whether the second Gram-Schmidt pass can be left out: h[0..nvec) are the
-// first-pass coefficients and h[nvec] = w.w.  After the first update
-// |w'|^2 = w.w - |h|^2; when |w'| >= eta |w| the first pass lost at most a
-// factor 1/eta of accuracy to cancellation and its result is kept (the
-// criterion of Daniel, Gragg, Kaufman & Stewart, Math. Comp. 30 (1976) 772,
-// with eta below their 1/sqrt(2)).  Sets *skip and, when set, h2 = 0 and
-// *beta = |w'| = sqrt(w.w - |h|^2) (relative error below eps / eta^2).
-__global__ void second_pass_test_kernel(const double *__restrict__ h, int nvec, double eta,
-                                        double *__restrict__ h2, int *__restrict__ skip,
-                                        double *__restrict__ beta) {
-  __shared__ int flag;
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < nvec; ++i) s = fma(h[i], h[i], s);
-    const double ww = h[nvec];
-    flag = (ww > 0.0 && ww - s >= eta * eta * ww) ? 1 : 0;
-    *skip = flag;
-    if (flag) *beta = sqrt(ww - s);
+// After the first pass, in one workgroup: the sums of its partials (h[0..
+// nvec) and h[nvec] = w.w) and whether the second Gram-Schmidt pass can be
+// left out.  After the first update |w'|^2 = w.w - |h|^2; when |w'| >= eta
+// |w| the first pass lost at most a factor 1/eta of accuracy to cancellation
+// and its result is kept (the criterion of Daniel, Gragg, Kaufman & Stewart,
+// Math. Comp. 30 (1976) 772, with eta below their 1/sqrt(2)).  Sets *skip
+// and, when set, *beta = |w'| = sqrt(w.w - |h|^2) (relative error below
+// eps / eta^2), column nvec - 1 of T and the breakdown flag.
+constexpr int kFirstPassThreads = 1024;
+__global__ void __launch_bounds__(kFirstPassThreads)
+    first_pass_kernel(const double *__restrict__ partial, int nvec, int G, double eta,
+                      double *__restrict__ h, int *__restrict__ skip, double *__restrict__ beta,
+                      double *__restrict__ flag, double *__restrict__ T, int ldt) {
+  __shared__ double sh[kFuseMax + 1];
+  __shared__ int keep;
+  for (int i = threadIdx.x >> 6; i <= nvec; i += kFirstPassThreads / 64) {
+    const double v = wave_partial_sum(partial + static_cast<uint64_t>(i) * G, G,
+                                      static_cast<int>(threadIdx.x & 63));
+    if ((threadIdx.x & 63) == 0) sh[i] = v;
   }
   __syncthreads();
-  if (flag)
-    for (int i = threadIdx.x; i < nvec; i += blockDim.x) h2[i] = 0.0;
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int i = 0; i < nvec; ++i) s = fma(sh[i], sh[i], s);
+    const double ww = sh[nvec];
+    keep = (ww > 0.0 && ww - s >= eta * eta * ww) ? 1 : 0;
+    *skip = keep;
+    if (keep) {
+      const double b = sqrt(ww - s);
+      *beta = b;
+      *flag = broke_down(b, sh[nvec - 1]);
+    }
+  }
+  __syncthreads();
+  const int j = nvec - 1;
+  for (int i = threadIdx.x; i <= nvec; i += kFirstPassThreads) {
+    h[i] = sh[i];
+    if (keep && i <= j) {
+      T[i * ldt + j] = sh[i];
+      T[j * ldt + i] = sh[i];
+    }
+  }
 }
 
-// v[r] = w[r] / (*beta) (beta == 0 -> zero vector); nothing when skip is
-// given and set (sub_norm_kernel stored v already)
+// After a second pass (nothing when *skip): the norm from its partials, v =
+// w / norm, and from the first workgroup beta, column j of T (h1 + h2) and
+// the breakdown flag.
+template <class VT>
+__global__ void __launch_bounds__(kBlock)
+    second_pass_store_kernel(const double *__restrict__ w, const double *__restrict__ partial,
+                             int G, VT *__restrict__ v, uint64_t n, const int *__restrict__ skip,
+                             const double *__restrict__ h1, const double *__restrict__ h2, int j,
+                             double *__restrict__ beta, double *__restrict__ flag,
+                             double *__restrict__ T, int ldt) {
+  if (*skip) return;
+  __shared__ double sb;
+  if (threadIdx.x < 64) {
+    const double ww = wave_partial_sum(partial, G, static_cast<int>(threadIdx.x));
+    if (threadIdx.x == 0) sb = sqrt(ww);
+  }
+  __syncthreads();
+  const double b = sb;
+  if (blockIdx.x == 0) {
+    const int i = static_cast<int>(threadIdx.x);
+    if (i <= j) {
+      const double t = h1[i] + h2[i];
+      T[i * ldt + j] = t;
+      T[j * ldt + i] = t;
+      if (i == j) *flag = broke_down(b, t);
+    }
+    if (i == 0) *beta = b;
+  }
+  const double inv = b > 0.0 ? 1.0 / b : 0.0;
+  for (uint64_t r = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x; r < n;
+       r += static_cast<uint64_t>(gridDim.x) * kBlock)
+    v[r] = static_cast<VT>(w[r] * inv);
+}
+
+// v[r] = w[r] / (*beta) (beta == 0 -> zero vector)
 template <class VT>
 __global__ void __launch_bounds__(kBlock)
     scale_store_kernel(const double *__restrict__ w, const double *__restrict__ beta,
-                       VT *__restrict__ v, uint64_t n, const int *__restrict__ skip = nullptr) {
-  if (skip && *skip) return;
+                       VT *__restrict__ v, uint64_t n) {
   const double b = *beta;
   const double inv = b > 0.0 ? 1.0 / b : 0.0;
   for (uint64_t r = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x; r < n;
@@ -358,25 +439,18 @@ __global__ void __launch_bounds__(kBlock)
     v[r] = static_cast<VT>(w[r] * inv);
 }
 
-__global__ void sqrt_inplace_kernel(double *v, const int *__restrict__ skip = nullptr) {
-  if (skip && *skip) return;
-  v[0] = sqrt(v[0]);
-}
-
-// T[i*ldt + j] = T[j*ldt + i] = h[i], i <= j; beta store
-__global__ void store_column_kernel(const double *__restrict__ h, int j, double *__restrict__ T,
-                                    int ldt) {
-  const int i = threadIdx.x;
-  if (i <= j) {
-    T[i * ldt + j] = h[i];
-    T[j * ldt + i] = h[i];
-  }
-}
+__global__ void sqrt_inplace_kernel(double *v) { v[0] = sqrt(v[0]); }
 
 __global__ void __launch_bounds__(256)
     jacobi_eigh_kernel(const double *__restrict__ T, int ldt, int m, double *__restrict__ evals,
-                       double *__restrict__ S, int max_sweeps) {
+                       double *__restrict__ S, int max_sweeps,
+                       double *__restrict__ last = nullptr) {
   jacobi_eigh_device(T, ldt, m, evals, S, max_sweeps);
+  if (last) { // last component of every eigenvector, for the residual estimates
+    __syncthreads();
+    for (int i = threadIdx.x; i < m; i += kJacobiThreads)
+      last[i] = S[static_cast<uint64_t>(i) * m + m - 1];
+  }
 }
 
 constexpr int kMaxKeepOne = 32; // kept Ritz vectors of the one-vector restart
@@ -469,12 +543,14 @@ __global__ void __launch_bounds__(kBlock) convert_kernel(const A *__restrict__ a
 // parts (the projected matrix of a Hermitian operator is real symmetric in
 // this basis; the imaginary parts are rounding).
 __global__ void store_column2_kernel(const double *__restrict__ h1, const double *__restrict__ h2,
-                                     int j, double *__restrict__ T, int ldt, int stride) {
+                                     int j, double *__restrict__ T, int ldt, int stride,
+                                     const double *__restrict__ beta, double *__restrict__ flag) {
   const int i = threadIdx.x;
   if (i <= j) {
     const double v = h1[stride * i] + h2[stride * i];
     T[i * ldt + j] = v;
     T[j * ldt + i] = v;
+    if (i == j) *flag = broke_down(*beta, v);
   }
 }
 
@@ -489,6 +565,28 @@ __global__ void reset_projected_kernel(double *__restrict__ T, int ldt,
 
 double seconds_since(std::chrono::steady_clock::time_point t0) {
   return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+}
+
+// Pinned host blocks of 4 KB for what a phase reads back, kept for the next
+// phase or solve (as many as have been live at once).
+std::mutex g_pinned_mu;
+std::vector<double *> g_pinned;
+double *pinned_block() {
+  {
+    std::lock_guard<std::mutex> lk(g_pinned_mu);
+    if (!g_pinned.empty()) {
+      double *p = g_pinned.back();
+      g_pinned.pop_back();
+      return p;
+    }
+  }
+  void *p = nullptr;
+  SPINED_HIP(hipHostMalloc(&p, 4096));
+  return static_cast<double *>(p);
+}
+void pinned_release(double *p) {
+  std::lock_guard<std::mutex> lk(g_pinned_mu);
+  g_pinned.push_back(p);
 }
 
 struct PhaseResult {
@@ -508,15 +606,25 @@ template <class VT, bool C = false> struct Phase {
   uint64_t ne; // doubles (or floats) per vector
   int m, k, keep;
   hipStream_t s;
-  std::vector<DeviceBuffer<VT>> vecs;
+  std::vector<DeviceBuffer<VT>> vecs; // large vectors (pooled), or
+  DeviceBuffer<VT> slab;              // all of them in one allocation
+  std::vector<VT *> hp;               // vector i
   DeviceBuffer<VT *> vptr;
   DeviceBuffer<const double *> wptr;
-  DeviceBuffer<double> w, partial, h, T, theta, S, beta;
+  DeviceBuffer<double> w, partial, h, T, S;
+  // what the host reads after a projected solve, one block: beta[kMaxBasis +
+  // 1], breakdown flags[kMaxBasis], theta[kMaxBasis], last components
+  DeviceBuffer<double> report;
+  double *beta, *flag, *theta, *last;
+  static constexpr int kReport = 4 * kMaxBasis + 1;
+  double *host_report;
   DeviceBuffer<int> skip; // second Gram-Schmidt pass left out (FP64 phase)
-  std::vector<hipEvent_t> ev;
+  std::vector<hipEvent_t> ev; // pairs around the matvecs since the last harvest
+  size_t ev_used = 0;
   int64_t matvecs = 0;
   double matvec_seconds = 0.0;
   unsigned G;
+  size_t norm_row = 0;
   bool small;
   int mlast = 0; // size of the last projected problem (Ritz assembly)
   // checkpoint after every cp_every-th restart (spined_eigsh_options)
@@ -534,10 +642,19 @@ template <class VT, bool C = false> struct Phase {
     static_assert(!C || std::is_same<VT, double>::value, "complex vectors are stored in FP64");
     // FP64-sized pooled blocks for either storage type: the FP32 phase of a
     // mixed solve hands them on to the FP64 phase without a free/allocate
-    vecs.resize(m + 1);
-    for (auto &v : vecs) v.allocate_pooled(ne, ne * sizeof(double));
-    std::vector<VT *> hp(m + 1);
-    for (int i = 0; i <= m; ++i) hp[i] = vecs[i].ptr;
+    // (vectors below the pool's block size share one allocation: twenty-odd
+    // hipMalloc and hipFree calls took 1 ms of a small solve)
+    const bool pooled = ne * sizeof(double) >= kPoolMinBytes;
+    const uint64_t pitch = (ne + 31) / 32 * 32; // 128-byte lines of their own
+    if (pooled)
+      vecs.resize(m + 1);
+    else
+      slab.allocate(pitch * static_cast<uint64_t>(m + 1));
+    hp.resize(m + 1);
+    for (int i = 0; i <= m; ++i) {
+      if (pooled) vecs[i].allocate_pooled(ne, ne * sizeof(double));
+      hp[i] = pooled ? vecs[i].ptr : slab.ptr + pitch * static_cast<uint64_t>(i);
+    }
     vptr.allocate(m + 1);
     SPINED_HIP(hipMemcpy(vptr.ptr, hp.data(), sizeof(VT *) * (m + 1), hipMemcpyHostToDevice));
     w.allocate_pooled(ne);
@@ -546,43 +663,52 @@ template <class VT, bool C = false> struct Phase {
     SPINED_HIP(hipMemcpy(wptr.ptr, &wp, sizeof(wp), hipMemcpyHostToDevice));
     G = grid_for(ne, 2048);
     const int chunks = (m + 1 + kDotChunk - 1) / kDotChunk;
-    partial.allocate(static_cast<size_t>(chunks) * kDotChunk * G * (C ? 2 : 1));
+    // one row past the dots' for the norm of the fused passes
+    norm_row = static_cast<size_t>(std::max(chunks * kDotChunk, kFuseMax + 1)) * G * (C ? 2 : 1);
+    partial.allocate(norm_row + G);
     h.allocate(4 * kMaxBasis + 4);
     T.allocate(kMaxBasis * kMaxBasis);
-    theta.allocate(kMaxBasis);
     S.allocate(kMaxBasis * kMaxBasis);
-    beta.allocate(kMaxBasis + 1);
+    report.allocate(kReport);
+    beta = report.ptr;
+    flag = beta + kMaxBasis + 1;
+    theta = flag + kMaxBasis;
+    last = theta + kMaxBasis;
+    host_report = pinned_block();
     skip.allocate(1);
-    reset_projected_kernel<<<1, 256, 0, s>>>(T.ptr, kMaxBasis, theta.ptr, 0);
+    reset_projected_kernel<<<1, 256, 0, s>>>(T.ptr, kMaxBasis, theta, 0);
     SPINED_CHECK_LAUNCH();
     small = n <= (1u << 20);
   }
   ~Phase() {
+    (void)hipStreamSynchronize(s); // a copy into the pinned block may be under way
+    pinned_release(host_report);
     for (auto e : ev) (void)hipEventDestroy(e);
   }
+  Phase(const Phase &) = delete;
+  Phase &operator=(const Phase &) = delete;
 
   void matvec(const void *x, VecType xt, double *y) {
-    hipEvent_t a, b;
-    SPINED_HIP(hipEventCreate(&a));
-    SPINED_HIP(hipEventCreate(&b));
-    SPINED_HIP(hipEventRecord(a, s));
+    while (ev.size() < ev_used + 2) {
+      hipEvent_t e;
+      SPINED_HIP(hipEventCreate(&e));
+      ev.push_back(e);
+    }
+    SPINED_HIP(hipEventRecord(ev[ev_used], s));
     MatvecCall c{&op, xt, xt == VecType::C128 ? VecType::C128 : VecType::F64, x, y, n, s};
     launch_matvec(c);
-    SPINED_HIP(hipEventRecord(b, s));
-    ev.push_back(a);
-    ev.push_back(b);
+    SPINED_HIP(hipEventRecord(ev[ev_used + 1], s));
+    ev_used += 2;
     ++matvecs;
   }
 
   void harvest_events() {
     SPINED_HIP(hipStreamSynchronize(s));
-    for (size_t i = 0; i + 1 < ev.size(); i += 2) {
+    for (size_t i = 0; i < ev_used; i += 2) {
       float ms = 0.f;
       if (hipEventElapsedTime(&ms, ev[i], ev[i + 1]) == hipSuccess) matvec_seconds += ms * 1e-3;
-      (void)hipEventDestroy(ev[i]);
-      (void)hipEventDestroy(ev[i + 1]);
     }
-    ev.clear();
+    ev_used = 0;
   }
 
   // real dots over `len` elements (default: the whole vector, ne)
@@ -639,38 +765,36 @@ template <class VT, bool C = false> struct Phase {
 
   // v_0 from an FP64 start vector in w (normalised here)
   void set_start_from_w() {
-    norm_w(beta.ptr);
-    scale_store_kernel<VT><<<G, kBlock, 0, s>>>(w.ptr, beta.ptr, vecs[0].ptr, ne);
+    norm_w(beta);
+    scale_store_kernel<VT><<<G, kBlock, 0, s>>>(w.ptr, beta, hp[0], ne);
     SPINED_CHECK_LAUNCH();
   }
 
-  // Classical Gram-Schmidt against V[0..nvec) (real vectors, nvec <=
-  // kFuseMax) and the norm of the result: dots with w.w; update + dots
-  // (the second pass); update + norm.  The second pass is left out on the
-  // device (no host round trip) when the first update loses little to
-  // cancellation (second_pass_test_kernel); the norm is then w.w - |h|^2
-  // and the update writes the next basis vector vnext = w' / |w'| itself
-  // (the caller's scale_store_kernel, given skip, does nothing).  Complex
-  // vectors take reorth() and norm_w().
-  void reorth_norm_fused(int nvec, double *h1, double *h2, double *norm_out, VT *vnext) {
+  // Classical Gram-Schmidt of w against V[0..j] (real vectors, j < kFuseMax),
+  // column j of T, beta_j and v_{j+1}: dots with w.w; their sums and the test
+  // for a second pass (first_pass_kernel); update + dots (the second pass);
+  // update and norm, or with one pass the next vector itself; after a second
+  // pass the next vector.  The second pass is decided on the device (no host
+  // round trip): its kernels read the flag and return.
+  void reorth_store_fused(int j, double *h1, double *h2) {
+    const int nvec = j + 1;
     // register width: the smallest multiple of 8 holding nvec vectors (the
     // slots past nvec still issue loads, of V[0])
     const int nq = (nvec + 7) / 8 * 8;
+    double *norm_part = partial.ptr + norm_row;
     auto passes = [&](auto width) {
       constexpr int NQ = decltype(width)::value;
       dot_ww_kernel<VT, NQ><<<G, kBlock, 0, s>>>(vptr.ptr, nvec, w.ptr, n, partial.ptr);
       SPINED_CHECK_LAUNCH();
-      reduce_partials_kernel<<<nvec + 1, kBlock, 0, s>>>(partial.ptr, nvec + 1, G, h1, 0);
-      SPINED_CHECK_LAUNCH();
-      second_pass_test_kernel<<<1, 64, 0, s>>>(h1, nvec, kSecondPassEta, h2, skip.ptr, norm_out);
+      first_pass_kernel<<<1, kFirstPassThreads, 0, s>>>(partial.ptr, nvec, G, kSecondPassEta, h1,
+                                                        skip.ptr, beta + j, flag + j, T.ptr,
+                                                        kMaxBasis);
       SPINED_CHECK_LAUNCH();
       sub_dot_kernel<VT, NQ>
           <<<G, kBlock, 0, s>>>(vptr.ptr, nvec, h1, w.ptr, n, partial.ptr, skip.ptr);
       SPINED_CHECK_LAUNCH();
-      reduce_partials_kernel<<<nvec, kBlock, 0, s>>>(partial.ptr, nvec, G, h2, 0, skip.ptr);
-      SPINED_CHECK_LAUNCH();
-      sub_norm_kernel<VT, NQ><<<G, kBlock, 0, s>>>(vptr.ptr, nvec, h2, w.ptr, n, partial.ptr,
-                                                   h1, skip.ptr, vnext, norm_out);
+      sub_norm_kernel<VT, NQ><<<G, kBlock, 0, s>>>(vptr.ptr, nvec, partial.ptr, h2, w.ptr, n,
+                                                   norm_part, h1, skip.ptr, hp[j + 1], beta + j);
       SPINED_CHECK_LAUNCH();
     };
     if (nq <= 8)
@@ -681,51 +805,44 @@ template <class VT, bool C = false> struct Phase {
       passes(std::integral_constant<int, 24>{});
     else
       passes(std::integral_constant<int, kFuseMax>{});
-    reduce_partials_kernel<<<1, kBlock, 0, s>>>(partial.ptr, 1, G, norm_out, 0, skip.ptr);
-    SPINED_CHECK_LAUNCH();
-    sqrt_inplace_kernel<<<1, 1, 0, s>>>(norm_out, skip.ptr);
+    second_pass_store_kernel<VT><<<G, kBlock, 0, s>>>(w.ptr, norm_part, G, hp[j + 1], n, skip.ptr,
+                                                      h1, h2, j, beta + j, flag + j, T.ptr,
+                                                      kMaxBasis);
     SPINED_CHECK_LAUNCH();
   }
 
-  void step(int j, uint64_t seed_breakdown) {
-    matvec(vecs[j].ptr,
+  void step(int j) {
+    matvec(hp[j],
            C ? VecType::C128 : (std::is_same<VT, float>::value ? VecType::F32 : VecType::F64),
            w.ptr);
     double *h1 = h.ptr, *h2 = h.ptr + 2 * kMaxBasis + 2;
-    const bool fused = !C && j + 1 <= kFuseMax;
-    if (fused) {
-      if constexpr (!C) reorth_norm_fused(j + 1, h1, h2, beta.ptr + j, vecs[j + 1].ptr);
-    } else {
-      reorth(j + 1, h1, h2);
-      norm_w(beta.ptr + j);
-    }
-    store_column2_kernel<<<1, kMaxBasis, 0, s>>>(h1, h2, j, T.ptr, kMaxBasis, C ? 2 : 1);
-    SPINED_CHECK_LAUNCH();
-    if (small) {
-      // breakdown guard (invariant subspace): continue with a random vector
-      double bj = 0.0, tj = 0.0;
-      SPINED_HIP(hipMemcpyAsync(&bj, beta.ptr + j, 8, hipMemcpyDeviceToHost, s));
-      SPINED_HIP(hipMemcpyAsync(&tj, T.ptr + j * kMaxBasis + j, 8, hipMemcpyDeviceToHost, s));
-      SPINED_HIP(hipStreamSynchronize(s));
-      if (bj <= 1e-12 * std::max(1.0, std::fabs(tj)) && j + 1 < static_cast<int>(n)) {
-        launch_random_fill(w.ptr, ne, seed_breakdown + 7919u * (j + 1), s);
-        double *g1 = h.ptr, *g2 = h.ptr + 2 * kMaxBasis + 2; // scratch (column already stored)
-        reorth(j + 1, g1, g2);
-        double nb = 0.0;
-        norm_w(beta.ptr + kMaxBasis);
-        SPINED_HIP(hipMemcpyAsync(&nb, beta.ptr + kMaxBasis, 8, hipMemcpyDeviceToHost, s));
-        SPINED_HIP(hipStreamSynchronize(s));
-        scale_store_kernel<VT><<<G, kBlock, 0, s>>>(w.ptr, beta.ptr + kMaxBasis, vecs[j + 1].ptr, ne);
-        SPINED_CHECK_LAUNCH();
-        const double zero = 0.0;
-        SPINED_HIP(hipMemcpyAsync(beta.ptr + j, &zero, 8, hipMemcpyHostToDevice, s));
-        SPINED_HIP(hipStreamSynchronize(s));
+    if constexpr (!C) {
+      if (j + 1 <= kFuseMax) {
+        reorth_store_fused(j, h1, h2);
         return;
       }
     }
-    scale_store_kernel<VT><<<G, kBlock, 0, s>>>(w.ptr, beta.ptr + j, vecs[j + 1].ptr, ne,
-                                                fused ? skip.ptr : nullptr);
+    reorth(j + 1, h1, h2);
+    norm_w(beta + j);
+    store_column2_kernel<<<1, kMaxBasis, 0, s>>>(h1, h2, j, T.ptr, kMaxBasis, C ? 2 : 1, beta + j,
+                                                 flag + j);
     SPINED_CHECK_LAUNCH();
+    scale_store_kernel<VT><<<G, kBlock, 0, s>>>(w.ptr, beta + j, hp[j + 1], ne);
+    SPINED_CHECK_LAUNCH();
+  }
+
+  // Breakdown at step j (invariant subspace): v_{j+1} becomes a random vector
+  // orthogonal to the basis, beta_j zero.
+  void restart_random(int j, uint64_t seed_breakdown) {
+    launch_random_fill(w.ptr, ne, seed_breakdown + 7919u * (j + 1), s);
+    double *g1 = h.ptr, *g2 = h.ptr + 2 * kMaxBasis + 2; // scratch (column already stored)
+    reorth(j + 1, g1, g2);
+    norm_w(beta + kMaxBasis);
+    scale_store_kernel<VT><<<G, kBlock, 0, s>>>(w.ptr, beta + kMaxBasis, hp[j + 1], ne);
+    SPINED_CHECK_LAUNCH();
+    const double zero = 0.0;
+    SPINED_HIP(hipMemcpyAsync(beta + j, &zero, 8, hipMemcpyHostToDevice, s));
+    SPINED_HIP(hipStreamSynchronize(s));
   }
 
   // Runs cycles until the k lowest estimates are <= tol, the matvec budget is
@@ -736,52 +853,72 @@ template <class VT, bool C = false> struct Phase {
     int j0 = 0;
     double best = 1e300;
     int stalled = 0;
-    std::vector<double> th(m), Sh(static_cast<size_t>(m) * m);
     // Convergence is also checked inside a cycle (on the leading block of T)
     // so that a good start vector is not held back to a restart boundary:
-    // every step when a matvec is expensive, every 4th otherwise.
+    // every step when a matvec is expensive, every 4th otherwise, and there
+    // only when the last estimate was within kFarEstimate of the target (a
+    // check is as long as two steps, and four steps gain less than that).
     const int check_every = n >= (1u << 20) ? 1 : 4;
-    // solve the leading msz x msz projected problem; estimates of the k lowest
+    constexpr double kFarEstimate = 1e5;
+    int checked = 0; // steps whose breakdown flag has been read
+    // Solves the leading msz x msz projected problem; estimates of the k
+    // lowest.  Returns the first unchecked step that broke down before the
+    // last one (its followers are then void), or -1.
     auto project = [&](int msz, double &worst, int &nconv) {
-      jacobi_eigh_kernel<<<1, 256, 0, s>>>(T.ptr, kMaxBasis, msz, theta.ptr, S.ptr, 40);
+      jacobi_eigh_kernel<<<1, 256, 0, s>>>(T.ptr, kMaxBasis, msz, theta, S.ptr, 40, last);
       SPINED_CHECK_LAUNCH();
-      double bm = 0.0;
-      SPINED_HIP(hipMemcpyAsync(th.data(), theta.ptr, 8 * msz, hipMemcpyDeviceToHost, s));
-      SPINED_HIP(hipMemcpyAsync(Sh.data(), S.ptr, 8ull * msz * msz, hipMemcpyDeviceToHost, s));
-      SPINED_HIP(hipMemcpyAsync(&bm, beta.ptr + (msz - 1), 8, hipMemcpyDeviceToHost, s));
+      SPINED_HIP(hipMemcpyAsync(host_report, report.ptr, sizeof(double) * kReport,
+                                hipMemcpyDeviceToHost, s));
       SPINED_HIP(hipStreamSynchronize(s));
-      res.theta.assign(th.begin(), th.begin() + k);
+      const double *hb = host_report, *hf = hb + kMaxBasis + 1;
+      const double *ht = hf + kMaxBasis, *hl = ht + kMaxBasis;
+      double bm = hb[msz - 1];
+      if (small) {
+        for (int i = checked; i < msz; ++i) {
+          if (hf[i] == 0.0 || i + 1 >= static_cast<int>(n)) continue;
+          restart_random(i, seed);
+          checked = i + 1;
+          if (i + 1 < msz) return i;
+          bm = 0.0;
+        }
+        checked = msz;
+      }
+      res.theta.assign(ht, ht + k);
       res.est.resize(k);
       worst = 0.0;
       nconv = 0;
       for (int i = 0; i < k; ++i) {
-        res.est[i] = std::fabs(bm * Sh[static_cast<size_t>(i) * msz + (msz - 1)]);
+        res.est[i] = std::fabs(bm * hl[i]);
         worst = std::max(worst, res.est[i]);
         if (res.est[i] <= tol) ++nconv;
       }
       mlast = msz;
+      return -1;
     };
+    double near = 0.0; // last estimate (0: none yet)
     for (;;) {
       double worst = 0.0;
       int nconv = 0;
-      bool early = false;
+      checked = j0;
       for (int j = j0; j < m; ++j) {
-        step(j, seed);
+        step(j);
         const int msz = j + 1;
-        if (msz < m && msz > k && (msz - j0) % check_every == 0) {
-          project(msz, worst, nconv);
-          if (nconv == k) {
-            early = true;
-            break;
-          }
+        const bool check = msz < m && msz > k && (msz - j0) % check_every == 0 &&
+                           (check_every == 1 || near <= kFarEstimate * tol);
+        if (!check && msz < m) continue;
+        const int broke = project(msz, worst, nconv);
+        if (broke >= 0) {
+          j = broke; // its successor vector is new: go on from there
+          continue;
         }
+        near = worst;
+        if (msz < m && nconv == k) break;
       }
-      if (!early) project(m, worst, nconv);
       harvest_events();
       ++res.cycles;
       if (verbose)
         log_line("phase %d cycle %d matvecs %lld theta0 %.15g est %.3e", phase_id, res.cycles,
-                 static_cast<long long>(matvecs), th[0], worst);
+                 static_cast<long long>(matvecs), res.theta[0], worst);
       int stop = 0;
       if (monitor) {
         spined_monitor_info info{matvecs, res.cycles, phase_id, nconv, k, res.theta.data(),
@@ -805,9 +942,8 @@ template <class VT, bool C = false> struct Phase {
       }
       // thick restart: keep the lowest `keep` Ritz vectors and v_m
       launch_restart<VT>(vptr.ptr, m, keep, S.ptr, ne, G, s);
-      SPINED_HIP(hipMemcpyAsync(vecs[keep].ptr, vecs[m].ptr, ne * sizeof(VT),
-                                hipMemcpyDeviceToDevice, s));
-      reset_projected_kernel<<<1, 256, 0, s>>>(T.ptr, kMaxBasis, theta.ptr, keep);
+      SPINED_HIP(hipMemcpyAsync(hp[keep], hp[m], ne * sizeof(VT), hipMemcpyDeviceToDevice, s));
+      reset_projected_kernel<<<1, 256, 0, s>>>(T.ptr, kMaxBasis, theta, keep);
       SPINED_CHECK_LAUNCH();
       j0 = keep;
       // V_0 now holds the lowest Ritz vector
@@ -815,7 +951,7 @@ template <class VT, bool C = false> struct Phase {
         SPINED_HIP(hipStreamSynchronize(s));
         spined_monitor_info info{matvecs, res.cycles, phase_id, nconv, k, res.theta.data(),
                                  res.est.data()};
-        cp_fn(vecs[0].ptr,
+        cp_fn(hp[0],
               C ? LS_COMPLEX128 : (std::is_same<VT, float>::value ? LS_FLOAT32 : LS_FLOAT64), n,
               &info, cp_ctx);
       }
