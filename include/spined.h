@@ -118,12 +118,12 @@ int spined_device_synchronize(void);
  * runtime), and copies / fills on the library stream (synchronous). */
 int spined_device_malloc(void **out, uint64_t bytes);
 int spined_device_free(void *ptr);
-/* The eigensolver keeps its vector blocks (those of 256 MiB or more) after a
- * solve and reuses them for the next solve or phase of the same size on the
- * device, and so does a dropped gather cache for its next build; this returns
- * them to the driver (hipFree).  The library also does
- * so by itself before any allocation the driver would refuse.  Call it
- * before allocating large device memory outside this library. */
+/* The library keeps device blocks that it no longer needs for its next calls:
+ * the eigensolver's vectors and a dropped gather cache's entries (blocks of
+ * 256 MiB or more), and up to 1 GiB of smaller temporaries per device.  This
+ * returns them to the driver (hipFree); the library does so by itself before
+ * any allocation the driver would refuse.  Call it before allocating large
+ * device memory outside this library. */
 int spined_device_release_pool(void);
 /* kind: 0 host->device, 1 device->host, 2 device->device */
 int spined_memcpy(void *dst, const void *src, uint64_t bytes, int kind);

@@ -5,6 +5,7 @@
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <vector>
 
 #include "handles.hpp"
@@ -47,6 +48,9 @@ struct PoolBlock {
 };
 std::mutex g_pool_mu;
 std::vector<PoolBlock> g_pool;
+// small blocks by (device, class size), newest last, and their bytes per device
+std::map<std::pair<int, size_t>, std::vector<void *>> g_small;
+std::map<int, size_t> g_small_bytes;
 
 void release_blocks(int device) {
   std::vector<void *> drop;
@@ -61,14 +65,26 @@ void release_blocks(int device) {
         ++i;
       }
     }
+    for (auto &kv : g_small) {
+      if (kv.first.first != device) continue;
+      drop.insert(drop.end(), kv.second.begin(), kv.second.end());
+      kv.second.clear();
+    }
+    g_small_bytes[device] = 0;
   }
   for (void *p : drop) (void)hipFree(p);
 }
 } // namespace
 
-void *device_alloc(size_t bytes, bool pooled) {
+size_t small_class(size_t bytes) {
+  size_t unit = 256;
+  while (unit * 8 < bytes) unit <<= 1; // classes 4, 5, 6, 7, 8 units wide
+  return (bytes + unit - 1) / unit * unit;
+}
+
+void *device_alloc(size_t bytes, Pool pool) {
   const int d = current_device();
-  if (pooled) {
+  if (pool == Pool::large) {
     std::lock_guard<std::mutex> lk(g_pool_mu);
     for (size_t i = 0; i < g_pool.size(); ++i) {
       if (g_pool[i].device == d && g_pool[i].bytes == bytes) {
@@ -77,6 +93,15 @@ void *device_alloc(size_t bytes, bool pooled) {
         g_pool.pop_back();
         return p;
       }
+    }
+  } else if (pool == Pool::small) {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    const auto it = g_small.find({d, bytes});
+    if (it != g_small.end() && !it->second.empty()) {
+      void *p = it->second.back();
+      it->second.pop_back();
+      g_small_bytes[d] -= bytes;
+      return p;
     }
   }
   void *p = nullptr;
@@ -95,12 +120,20 @@ void *device_alloc(size_t bytes, bool pooled) {
   return p;
 }
 
-void device_free(void *p, size_t bytes, bool pooled, int device) {
+void device_free(void *p, size_t bytes, Pool pool, int device) {
   if (!p) return;
-  if (pooled) {
+  if (pool != Pool::none) {
     std::lock_guard<std::mutex> lk(g_pool_mu);
-    g_pool.push_back(PoolBlock{device, bytes, p});
-    return;
+    if (pool == Pool::large) {
+      g_pool.push_back(PoolBlock{device, bytes, p});
+      return;
+    }
+    size_t &kept = g_small_bytes[device];
+    if (kept + bytes <= kSmallPoolBytes) {
+      kept += bytes;
+      g_small[{device, bytes}].push_back(p);
+      return;
+    }
   }
   (void)hipFree(p);
 }
@@ -114,6 +147,13 @@ size_t pool_bytes(size_t bytes) {
   for (const PoolBlock &b : g_pool)
     if (b.device == d && b.bytes == bytes) s += b.bytes;
   return s;
+}
+
+void copy_in(void *dst, const void *src, size_t bytes) {
+  if (bytes == 0) return;
+  hipStream_t s = stream();
+  SPINED_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+  SPINED_HIP(hipStreamSynchronize(s));
 }
 
 hipStream_t stream() {
@@ -572,7 +612,7 @@ int spined_device_synchronize(void) {
 int spined_device_malloc(void **out, uint64_t bytes) {
   return guarded([&] {
     if (!out) throw Error(LS_INVALID_ARGUMENT, "NULL argument");
-    *out = device_alloc(bytes ? bytes : 1, false);
+    *out = device_alloc(bytes ? bytes : 1, Pool::none);
   });
 }
 

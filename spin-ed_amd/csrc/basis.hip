@@ -588,7 +588,7 @@ void adopt_basis(Basis &b, uint64_t n, const uint64_t *reps) {
     throw Error(LS_NOT_IMPLEMENTED, "dimensions of 2^32 - 1 or more are not supported");
   validate_representatives(b, n, reps);
   b.reps.allocate(std::max<uint64_t>(n, 1));
-  if (n) SPINED_HIP(hipMemcpy(b.reps.ptr, reps, n * 8, hipMemcpyHostToDevice));
+  if (n) copy_in(b.reps.ptr, reps, n * 8);
   b.D = n;
   b.stab.allocate(std::max<uint64_t>(n, 1));
   // the list is the whole sector when each entry is a valid orbit minimum

@@ -369,15 +369,15 @@ template <class VT, int K> struct BlockPhase {
     blocks.resize(mb + 1);
     hptr.resize(mb + 1);
     for (int i = 0; i <= mb; ++i) {
-      blocks[i].allocate(n * K);
+      blocks[i].allocate_pooled(n * K); // 1 GB each on the 6x6 lattice
       hptr[i] = blocks[i].ptr;
     }
     vptr.allocate(mb + 1);
     upload_pointers();
-    W.allocate(n * K);
+    W.allocate_pooled(n * K);
     const double *wp = W.ptr;
     wptr.allocate(1);
-    SPINED_HIP(hipMemcpy(wptr.ptr, &wp, sizeof(wp), hipMemcpyHostToDevice));
+    copy_in(wptr.ptr, &wp, sizeof(wp));
     Gd = grid_for(n, 1024);
     partial.allocate(static_cast<size_t>(mb + 1) * K * K * Gd);
     C.allocate(2 * static_cast<size_t>(mb + 1) * K * K);

@@ -832,9 +832,9 @@ int spined_cnn_create(spined_cnn **out, const float *init_params) {
     c->m.v.allocate(spined::NPARAMS);
     c->m.grad.allocate(spined::NPARAMS);
     c->m.table.allocate(spined::kInferPrepWords);
-    SPINED_HIP(hipMemcpy(c->m.params.ptr, init_params, 4 * spined::NPARAMS, hipMemcpyHostToDevice));
-    SPINED_HIP(hipMemset(c->m.m.ptr, 0, 4 * spined::NPARAMS));
-    SPINED_HIP(hipMemset(c->m.v.ptr, 0, 4 * spined::NPARAMS));
+    spined::copy_in(c->m.params.ptr, init_params, 4 * spined::NPARAMS);
+    SPINED_HIP(hipMemsetAsync(c->m.m.ptr, 0, 4 * spined::NPARAMS, spined::stream()));
+    SPINED_HIP(hipMemsetAsync(c->m.v.ptr, 0, 4 * spined::NPARAMS, spined::stream()));
     *out = c;
   });
 }
@@ -844,14 +844,16 @@ void spined_cnn_destroy(spined_cnn *c) { delete c; }
 int spined_cnn_get_params(const spined_cnn *c, float *out) {
   return spined::guarded([&] {
     if (!c || !out) throw Error(LS_INVALID_ARGUMENT, "NULL argument");
-    SPINED_HIP(hipMemcpy(out, c->m.params.ptr, 4 * spined::NPARAMS, hipMemcpyDeviceToHost));
+    SPINED_HIP(hipMemcpyAsync(out, c->m.params.ptr, 4 * spined::NPARAMS, hipMemcpyDeviceToHost,
+                              spined::stream()));
+    SPINED_HIP(hipStreamSynchronize(spined::stream()));
   });
 }
 
 int spined_cnn_set_params(spined_cnn *c, const float *in) {
   return spined::guarded([&] {
     if (!c || !in) throw Error(LS_INVALID_ARGUMENT, "NULL argument");
-    SPINED_HIP(hipMemcpy(c->m.params.ptr, in, 4 * spined::NPARAMS, hipMemcpyHostToDevice));
+    spined::copy_in(c->m.params.ptr, in, 4 * spined::NPARAMS);
   });
 }
 

@@ -41,20 +41,28 @@ void log_line(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 hipStream_t stream();
 int current_device();
 
-// Pool of large device blocks (at least kPoolMinBytes).  The eigensolver's
-// vectors (6.9 GB each at D = 8.6e8, dozens per solve) and the entry blocks
-// of dropped gather caches go back to the pool instead of to hipFree, which
-// unmaps them page by page, and the next allocation of the same size on the
-// device takes them again.  Every library kernel runs on the device's
-// library stream, so a reused block is only touched after the work that
-// used it before.  An allocation that the driver refuses drops the gather
-// caches not in use (into the pool), returns the pooled blocks of the
-// device and retries once.
+// Pools of device blocks.  Every library kernel and copy runs on the device's
+// library stream, so a block that is handed on is only touched after the work
+// that used it before; host copies into a block go through that stream too
+// (copy_in).  Large blocks (allocate_pooled, at least kPoolMinBytes): the
+// eigensolver's vectors (6.9 GB each at D = 8.6e8, dozens per solve) and the
+// entry blocks of dropped gather caches, of exactly the size asked for,
+// instead of hipFree, which unmaps them page by page.  Small blocks
+// (everything else below kPoolMinBytes): rounded up to a quarter of a power
+// of two, at most kSmallPoolBytes of them kept per device; a hipMalloc and
+// hipFree pair costs 20 to 200 us.  An allocation that the driver refuses
+// drops the gather caches not in use (into the pool), returns the pooled
+// blocks of the device and retries once.
 constexpr size_t kPoolMinBytes = size_t(256) << 20;
-void *device_alloc(size_t bytes, bool pooled); // throws Error(LS_OUT_OF_MEMORY)
-void device_free(void *p, size_t bytes, bool pooled, int device);
+constexpr size_t kSmallPoolBytes = size_t(1) << 30;
+enum class Pool { none, large, small };
+size_t small_class(size_t bytes);              // size of the small block for `bytes`
+void *device_alloc(size_t bytes, Pool pool);   // throws Error(LS_OUT_OF_MEMORY)
+void device_free(void *p, size_t bytes, Pool pool, int device);
 void pool_release_device();                    // hipFree the current device's pooled blocks
-size_t pool_bytes(size_t bytes);               // pooled bytes in blocks of this size (current device)
+size_t pool_bytes(size_t bytes);               // pooled bytes in large blocks of this size (current device)
+// Host -> device copy of `bytes`, complete on return, in stream order.
+void copy_in(void *dst, const void *src, size_t bytes);
 
 // Device buffer with RAII release (any thread).  allocate_pooled(count,
 // bytes) takes a block of max(count * sizeof(T), bytes) bytes from the pool.
@@ -62,7 +70,7 @@ template <class T> struct DeviceBuffer {
   T *ptr = nullptr;
   size_t n = 0;
   size_t cap = 0;      // bytes of the block
-  bool pooled = false;
+  Pool pooled = Pool::none;
   int dev = 0;         // device of a pooled block
   DeviceBuffer() = default;
   explicit DeviceBuffer(size_t count) { allocate(count); }
@@ -102,10 +110,11 @@ template <class T> struct DeviceBuffer {
 private:
   void take(size_t count, size_t bytes, bool pool) {
     release();
-    const size_t b = std::max(count * sizeof(T), bytes);
+    size_t b = std::max(count * sizeof(T), bytes);
     if (b) {
-      pooled = pool && b >= kPoolMinBytes;
-      if (pooled) dev = current_device();
+      pooled = b < kPoolMinBytes ? Pool::small : pool ? Pool::large : Pool::none;
+      if (pooled == Pool::small) b = small_class(b);
+      if (pooled != Pool::none) dev = current_device();
       ptr = static_cast<T *>(device_alloc(b, pooled));
       cap = b;
     }

@@ -234,7 +234,7 @@ void detect_torus(const Group &g, int n, OrbitTables &t) {
 template <class T> void upload(DeviceBuffer<T> &d, const std::vector<T> &h) {
   d.allocate(std::max<size_t>(h.size(), 1));
   if (!h.empty())
-    SPINED_HIP(hipMemcpy(d.ptr, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+    copy_in(d.ptr, h.data(), h.size() * sizeof(T));
 }
 } // namespace
 

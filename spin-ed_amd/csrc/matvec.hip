@@ -942,6 +942,13 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
   const Basis &b = *op.basis;
   const int units = unit_count(op.tables);
   if (gc.request == 0 || b.D > (1ull << 31) || units > 65535) return false;
+  // nothing is built under stream capture: its kernels would only run at a replay
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  SPINED_HIP(hipStreamIsCapturing(s, &cap));
+  if (cap != hipStreamCaptureStatusNone) {
+    if (gc.request > 0) throw Error(LS_DEVICE_ERROR, "gather cache: not built under stream capture");
+    return false;
+  }
   struct Building {
     std::atomic<bool> &f;
     explicit Building(std::atomic<bool> &x) : f(x) { f.store(true); }
@@ -1114,10 +1121,13 @@ bool try_split(const MatvecCall &m, const Ctx &c) {
     }
     if (!op.split_dlow.ptr) {
       if (m.no_alloc) return false;
-      op.split_dlow.allocate(size_t(1) << l);
+      // published once it is computed (an error under stream capture)
+      DeviceBuffer<double> d(size_t(1) << l);
       split_dlow_kernel<<<grid_for(uint64_t(1) << l), kBlock, 0, m.stream>>>(
-          b.split_args(b.split), c.bd, op.split_dlow.ptr);
+          b.split_args(b.split), c.bd, d.ptr);
       SPINED_CHECK_LAUNCH();
+      SPINED_HIP(hipStreamSynchronize(m.stream));
+      op.split_dlow = std::move(d);
     }
   }
   if (m.xt == VT::F64)
@@ -1271,8 +1281,8 @@ const PhaseTable &phase_table(const Basis &b, bool no_alloc = false) {
   for (int p = 0; p < L; ++p) phase_values(p, L, c[p], s[p]);
   t->cos_t.allocate(L);
   t->sin_t.allocate(L);
-  SPINED_HIP(hipMemcpy(t->cos_t.ptr, c.data(), 8 * L, hipMemcpyHostToDevice));
-  SPINED_HIP(hipMemcpy(t->sin_t.ptr, s.data(), 8 * L, hipMemcpyHostToDevice));
+  copy_in(t->cos_t.ptr, c.data(), 8 * L);
+  copy_in(t->sin_t.ptr, s.data(), 8 * L);
   t->L = L;
   cache.emplace_back(std::make_pair(dev, L), std::move(t));
   return *cache.back().second;

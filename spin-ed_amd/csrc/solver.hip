@@ -656,11 +656,11 @@ template <class VT, bool C = false> struct Phase {
       hp[i] = pooled ? vecs[i].ptr : slab.ptr + pitch * static_cast<uint64_t>(i);
     }
     vptr.allocate(m + 1);
-    SPINED_HIP(hipMemcpy(vptr.ptr, hp.data(), sizeof(VT *) * (m + 1), hipMemcpyHostToDevice));
+    copy_in(vptr.ptr, hp.data(), sizeof(VT *) * (m + 1));
     w.allocate_pooled(ne);
     const double *wp = w.ptr;
     wptr.allocate(1);
-    SPINED_HIP(hipMemcpy(wptr.ptr, &wp, sizeof(wp), hipMemcpyHostToDevice));
+    copy_in(wptr.ptr, &wp, sizeof(wp));
     G = grid_for(ne, 2048);
     const int chunks = (m + 1 + kDotChunk - 1) / kDotChunk;
     // one row past the dots' for the norm of the fused passes
