@@ -331,6 +331,90 @@ __global__ void __launch_bounds__(64)
   }
 }
 
+// Forward pass of a training step (pre-activations stored): cnn_forward_kernel
+// with kFwdWaves waves per 16 samples, each taking every kFwdWaves-th position
+// of a layer.  A batch of 2,048 samples is 128 workgroups, so one wave each
+// left the chip idle and ran every position in turn (33 us; now 21).  The
+// layer-3 activations meet in LDS and the first wave adds them in position
+// order: the outputs are those of the one-wave kernel bit for bit.
+constexpr int kFwdWaves = 8;
+__global__ void __launch_bounds__(64 * kFwdWaves)
+    cnn_forward_store_kernel(CnnArgs c, const uint64_t *__restrict__ states,
+                             float *__restrict__ out_a, float *__restrict__ out_t,
+                             float *__restrict__ z_store) {
+  extern __shared__ __attribute__((aligned(16))) __bf16 lds[];
+  const int n = c.n;
+  __bf16 *h2 = lds, *h1 = lds + 16 * n * CH;
+  float *act3 = reinterpret_cast<float *>(h1); // [16][n][16], over h1 (read no more) and beyond
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, s = lane & 15, g = lane >> 4;
+  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * 16;
+  const uint64_t sample = base + s;
+  const uint64_t state = sample < c.count ? states[sample] : 0;
+  const float *P = c.params;
+  const size_t per = static_cast<size_t>(n) * CH;
+  const size_t padded = (c.count + 15) / 16 * 16;
+  float *z1 = z_store + base * per;
+  float *z2 = z_store + padded * per + base * per;
+  float *z3 = z_store + 2 * padded * per + base * per;
+  float bias[4];
+  {
+    const bf16x8 a = load_first_weights(P + OFF_W1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bias[r] = P[OFF_B1 + 4 * g + r];
+    for (int pos = wv; pos < n; pos += kFwdWaves) {
+      floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+      acc = mfma(a, spin_fragment(state, n, pos), acc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] += bias[r];
+      store4_f32(z1, n, pos, acc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = gelu_f(acc[r]);
+      store4(h1, n, pos, acc);
+    }
+  }
+  auto conv_layer = [&](const __bf16 *in, int off_w, int off_b, float *z, auto &&put) {
+    bf16x8 a[3];
+    load_conv_weights(P + off_w, false, a);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bias[r] = P[off_b + 4 * g + r];
+    for (int pos = wv; pos < n; pos += kFwdWaves) {
+      floatx4 acc = conv_at(a, in, n, pos);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] += bias[r];
+      store4_f32(z, n, pos, acc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = gelu_f(acc[r]);
+      put(pos, acc);
+    }
+  };
+  __syncthreads();
+  conv_layer(h1, OFF_W2, OFF_B2, z2, [&](int pos, floatx4 v) { store4(h2, n, pos, v); });
+  __syncthreads();
+  conv_layer(h2, OFF_W3, OFF_B3, z3, [&](int pos, floatx4 v) { store4_f32(act3, n, pos, v); });
+  __syncthreads();
+  if (wv != 0) return;
+  float f[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int pos = 0; pos < n; ++pos) {
+    const floatx4 v = load4_f32(act3, n, pos);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f[r] += v[r];
+  }
+  float pa = 0.f, pt = 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    pa += P[OFF_U + 4 * g + r] * f[r];
+    pt += P[OFF_V + 4 * g + r] * f[r];
+  }
+  pa += __shfl_xor(pa, 16, 64);
+  pa += __shfl_xor(pa, 32, 64);
+  pt += __shfl_xor(pt, 16, 64);
+  pt += __shfl_xor(pt, 32, 64);
+  if (g == 0 && sample < c.count) {
+    out_a[sample] = pa + P[OFF_U0];
+    out_t[sample] = pt + P[OFF_V0];
+  }
+}
+
 // Streaming inference (no stored pre-activations, n >= kInferMinN): the
 // forward kernel's network (same BF16 operands; the polynomial GELU gates
 // in layers 2 and 3; MFMA sums that start from the bias instead of adding
@@ -506,63 +590,56 @@ __global__ void __launch_bounds__(64)
   }
 }
 
-// Weight gradient of one conv layer: C_d[co][ci] += sum_slots dz[slot][co] *
-// h[slot shifted by d][ci]; 32 (sample, position) slots per MFMA.
-// Layer 1 (first = true): C[co][d] with h = spins.
+// Weight gradient of one tap of a conv layer: C_d[co][ci] += sum_slots
+// dz[slot][co] * h[slot shifted by d][ci]; 32 (sample, position) slots per
+// MFMA.  Layer 1 (first = true): C[co][d] with h = spins, every tap at once.
+// dbias: this lane's share of the bias gradient.
 __device__ inline void weight_grad(const __bf16 *dz, const __bf16 *h, const uint64_t *st, int n,
-                                   bool first, floatx4 (&cacc)[KW], float &dbias) {
+                                   bool first, int d, floatx4 &cacc, float &dbias) {
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int nslots = 16 * n;
+  // sample and position of this lane's first slot of the step; the next
+  // step's is 32 slots on (no division per slot)
+  int s0 = (8 * g) / n, p0 = (8 * g) % n;
   for (int c0 = 0; c0 < nslots; c0 += 32) {
-    bf16x8 a;
-    int ss[8], pp[8];
+    bf16x8 a, b;
+    int ss = s0, pp = p0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int slot = c0 + 8 * g + j;
-      const bool ok = slot < nslots;
-      ss[j] = ok ? slot / n : 0;
-      pp[j] = ok ? slot % n : 0;
-      const float v = ok ? static_cast<float>(dz[(static_cast<size_t>(ss[j]) * n + pp[j]) * CH + col]) : 0.0f;
+      const bool ok = ss < 16;
+      const float v = ok ? static_cast<float>(dz[(static_cast<size_t>(ss) * n + pp) * CH + col]) : 0.0f;
       a[j] = static_cast<__bf16>(v);
       dbias += v;
-      if (!ok) ss[j] = -1;
+      float u = 0.0f;
+      if (ok && (!first || col < KW)) {
+        int p = pp + (first ? col : d) - 2;
+        p = p < 0 ? p + n : (p >= n ? p - n : p);
+        u = first ? (((st[ss] >> p) & 1) ? 1.0f : -1.0f)
+                  : static_cast<float>(h[(static_cast<size_t>(ss) * n + p) * CH + col]);
+      }
+      b[j] = static_cast<__bf16>(u);
+      ++pp;
+      if (pp == n) {
+        pp = 0;
+        ++ss;
+      }
     }
-    if (first) {
-      bf16x8 b;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float v = 0.0f;
-        if (ss[j] >= 0 && col < KW) {
-          int p = pp[j] + col - 2;
-          p = p < 0 ? p + n : (p >= n ? p - n : p);
-          v = ((st[ss[j]] >> p) & 1) ? 1.0f : -1.0f;
-        }
-        b[j] = static_cast<__bf16>(v);
-      }
-      cacc[0] = mfma(a, b, cacc[0]);
-    } else {
-#pragma unroll
-      for (int d = 0; d < KW; ++d) {
-        bf16x8 b;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float v = 0.0f;
-          if (ss[j] >= 0) {
-            int p = pp[j] + d - 2;
-            p = p < 0 ? p + n : (p >= n ? p - n : p);
-            v = static_cast<float>(h[(static_cast<size_t>(ss[j]) * n + p) * CH + col]);
-          }
-          b[j] = static_cast<__bf16>(v);
-        }
-        cacc[d] = mfma(a, b, cacc[d]);
-      }
+    cacc = mfma(a, b, cacc);
+    p0 += 32;
+    while (p0 >= n) {
+      p0 -= n;
+      ++s0;
     }
   }
 }
 
-// Backward for one wave of 16 samples: per-wave partial gradients
-// (NPARAMS floats) of sum_s ga[s] a_s + gt[s] t_s.
-__global__ void __launch_bounds__(64)
+// Backward pass of 16 samples: kBwdWaves waves, one per tap of the weight
+// gradients; the data gradients and activations are split by position.  One
+// wave ran all of it in turn on half of the chip (2,048 samples of 30 sites: 151
+// us; now 69).
+// Every sum is formed by one wave in the order of the one-wave kernel.
+constexpr int kBwdWaves = KW;
+__global__ void __launch_bounds__(64 * kBwdWaves)
     cnn_backward_kernel(CnnArgs c, const uint64_t *__restrict__ states,
                         const float *__restrict__ z_store, const float *__restrict__ ga,
                         const float *__restrict__ gt, float *__restrict__ partial) {
@@ -572,11 +649,11 @@ __global__ void __launch_bounds__(64)
   __bf16 *bufA = lds, *bufB = lds + act, *bufC = lds + 2 * act;
   __shared__ uint64_t st[16];
   __shared__ float gsh[2][16];
-  const int lane = threadIdx.x, s = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, s = lane & 15, g = lane >> 4;
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * 16;
   const uint64_t sample = base + s;
   const bool valid = sample < c.count;
-  if (g == 0) {
+  if (threadIdx.x < 16) {
     st[s] = valid ? states[sample] : 0;
     gsh[0][s] = valid ? ga[sample] : 0.0f;
     gsh[1][s] = valid ? gt[sample] : 0.0f;
@@ -591,38 +668,28 @@ __global__ void __launch_bounds__(64)
   float *out = partial + static_cast<size_t>(blockIdx.x) * NPARAMS;
   const float gas = gsh[0][s], gts = gsh[1][s];
 
-  // heads and d3 = (ga u + gt v) gelu'(z3)  -> bufA; h2 = gelu(z2) -> bufB
-  float f[4] = {0.f, 0.f, 0.f, 0.f};
-  float coef[4];
+  // heads (the last wave: f is a sum over positions) and, by the others,
+  // d3 = (ga u + gt v) gelu'(z3) -> bufA; h2 = gelu(z2) -> bufB
+  if (wv == kBwdWaves - 1) {
+    float f[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int pos = 0; pos < n; ++pos) {
+      const floatx4 z = load4_f32(z3, n, pos);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) coef[r] = gas * P[OFF_U + 4 * g + r] + gts * P[OFF_V + 4 * g + r];
-  for (int pos = 0; pos < n; ++pos) {
-    floatx4 z = load4_f32(z3, n, pos), d;
+      for (int r = 0; r < 4; ++r) f[r] += gelu_f(z[r]);
+    }
+    // du[co] = sum_s ga[s] f[s][co]: reduce over the 16 samples of a lane group
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      f[r] += gelu_f(z[r]);
-      d[r] = valid ? coef[r] * gelu_grad_f(z[r]) : 0.0f;
+      float du = valid ? gas * f[r] : 0.0f, dv = valid ? gts * f[r] : 0.0f;
+      for (int off = 8; off > 0; off >>= 1) {
+        du += __shfl_xor(du, off, 64);
+        dv += __shfl_xor(dv, off, 64);
+      }
+      if (s == 0) {
+        out[OFF_U + 4 * g + r] = du;
+        out[OFF_V + 4 * g + r] = dv;
+      }
     }
-    store4(bufA, n, pos, d);
-    floatx4 z2v = load4_f32(z2, n, pos), h;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) h[r] = gelu_f(z2v[r]);
-    store4(bufB, n, pos, h);
-  }
-  // du[co] = sum_s ga[s] f[s][co]: reduce over the 16 samples of a lane group
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    float du = valid ? gas * f[r] : 0.0f, dv = valid ? gts * f[r] : 0.0f;
-    for (int off = 8; off > 0; off >>= 1) {
-      du += __shfl_xor(du, off, 64);
-      dv += __shfl_xor(dv, off, 64);
-    }
-    if (s == 0) {
-      out[OFF_U + 4 * g + r] = du;
-      out[OFF_V + 4 * g + r] = dv;
-    }
-  }
-  {
     float a0 = gas, t0 = gts;
     for (int off = 8; off > 0; off >>= 1) {
       a0 += __shfl_xor(a0, off, 64);
@@ -632,92 +699,81 @@ __global__ void __launch_bounds__(64)
       out[OFF_U0] = a0;
       out[OFF_V0] = t0;
     }
+  } else {
+    float coef[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) coef[r] = gas * P[OFF_U + 4 * g + r] + gts * P[OFF_V + 4 * g + r];
+    for (int pos = wv; pos < n; pos += kBwdWaves - 1) {
+      floatx4 z = load4_f32(z3, n, pos), d;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[r] = valid ? coef[r] * gelu_grad_f(z[r]) : 0.0f;
+      store4(bufA, n, pos, d);
+      floatx4 z2v = load4_f32(z2, n, pos), h;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) h[r] = gelu_f(z2v[r]);
+      store4(bufB, n, pos, h);
+    }
   }
   __syncthreads();
 
-  auto write_wgrad = [&](int off_w, int off_b, floatx4 (&cacc)[KW], float dbias, bool first) {
-    // cacc[d]: rows co = 4g + r, column = ci (or d for the first layer)
+  // this wave's tap of a layer's weight gradient; the first wave has the bias
+  auto wgrad = [&](const __bf16 *dz, const __bf16 *h, int off_w, int off_b) {
+    floatx4 cacc = {0.f, 0.f, 0.f, 0.f};
+    float db = 0.0f;
+    weight_grad(dz, h, st, n, false, wv, cacc, db);
     const int col = lane & 15;
+    // rows co = 4g + r, column = ci
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int co = 4 * g + r;
-      if (first) {
-        if (col < KW) out[off_w + co * KW + col] = cacc[0][r];
-      } else {
+    for (int r = 0; r < 4; ++r) out[off_w + ((4 * g + r) * CH + col) * KW + wv] = cacc[r];
+    // db holds this lane's share for channel `col` (A rows are co = col)
+    db += __shfl_xor(db, 16, 64);
+    db += __shfl_xor(db, 32, 64);
+    if (wv == 0 && g == 0) out[off_b + col] = db;
+  };
+  // dst = conv^T(d) * gelu'(z)
+  auto data_grad = [&](const __bf16 *d, int off_w, const float *z, __bf16 *dst) {
+    bf16x8 a[3];
+    load_conv_weights(P + off_w, true, a);
+    for (int pos = wv; pos < n; pos += kBwdWaves) {
+      floatx4 acc = conv_at(a, d, n, pos);
+      floatx4 zz = load4_f32(z, n, pos);
 #pragma unroll
-        for (int d = 0; d < KW; ++d) out[off_w + (co * CH + col) * KW + d] = cacc[d][r];
-      }
+      for (int r = 0; r < 4; ++r) acc[r] *= gelu_grad_f(zz[r]);
+      store4(dst, n, pos, acc);
     }
-    // bias: dbias holds this lane's share for channel `col` (A rows are co = col)
-    float b = dbias;
-    b += __shfl_xor(b, 16, 64);
-    b += __shfl_xor(b, 32, 64);
-    if (g == 0) out[off_b + col] = b;
   };
 
   // layer 3 weight gradient (dz = bufA, h = bufB)
-  {
-    floatx4 cacc[KW];
-#pragma unroll
-    for (int d = 0; d < KW; ++d) cacc[d] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float db = 0.0f;
-    weight_grad(bufA, bufB, st, n, false, cacc, db);
-    write_wgrad(OFF_W3, OFF_B3, cacc, db, false);
-  }
+  wgrad(bufA, bufB, OFF_W3, OFF_B3);
   __syncthreads();
-  // d2 = conv^T(d3) * gelu'(z2) -> bufC ; h1 = gelu(z1) -> bufB
-  {
-    bf16x8 a[3];
-    load_conv_weights(P + OFF_W3, true, a);
-    for (int pos = 0; pos < n; ++pos) {
-      floatx4 acc = conv_at(a, bufA, n, pos);
-      floatx4 z = load4_f32(z2, n, pos);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] *= gelu_grad_f(z[r]);
-      store4(bufC, n, pos, acc);
-    }
-  }
-  __syncthreads();
-  for (int pos = 0; pos < n; ++pos) {
+  // d2 -> bufC; h1 = gelu(z1) -> bufB
+  data_grad(bufA, OFF_W3, z2, bufC);
+  for (int pos = wv; pos < n; pos += kBwdWaves) {
     floatx4 z = load4_f32(z1, n, pos), h;
 #pragma unroll
     for (int r = 0; r < 4; ++r) h[r] = gelu_f(z[r]);
     store4(bufB, n, pos, h);
   }
   __syncthreads();
-  // layer 2 weight gradient (dz = bufC, h = bufB)
-  {
-    floatx4 cacc[KW];
-#pragma unroll
-    for (int d = 0; d < KW; ++d) cacc[d] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float db = 0.0f;
-    weight_grad(bufC, bufB, st, n, false, cacc, db);
-    write_wgrad(OFF_W2, OFF_B2, cacc, db, false);
-  }
+  // layer 2 weight gradient (dz = bufC, h = bufB); d1 -> bufA
+  wgrad(bufC, bufB, OFF_W2, OFF_B2);
+  data_grad(bufC, OFF_W2, z1, bufA);
   __syncthreads();
-  // d1 = conv^T(d2) * gelu'(z1) -> bufA
-  {
-    bf16x8 a[3];
-    load_conv_weights(P + OFF_W2, true, a);
-    for (int pos = 0; pos < n; ++pos) {
-      floatx4 acc = conv_at(a, bufC, n, pos);
-      floatx4 z = load4_f32(z1, n, pos);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] *= gelu_grad_f(z[r]);
-      store4(bufA, n, pos, acc);
-    }
-  }
-  __syncthreads();
-  // layer 1 weight gradient (dz = bufA, input spins)
-  {
-    floatx4 cacc[KW];
-#pragma unroll
-    for (int d = 0; d < KW; ++d) cacc[d] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // layer 1 weight gradient (dz = bufA, input spins): one product for all taps
+  if (wv == 0) {
+    floatx4 cacc = {0.f, 0.f, 0.f, 0.f};
     float db = 0.0f;
-    weight_grad(bufA, nullptr, st, n, true, cacc, db);
-    write_wgrad(OFF_W1, OFF_B1, cacc, db, true);
+    weight_grad(bufA, nullptr, st, n, true, 0, cacc, db);
+    const int col = lane & 15;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (col < KW) out[OFF_W1 + (4 * g + r) * KW + col] = cacc[r];
+    db += __shfl_xor(db, 16, 64);
+    db += __shfl_xor(db, 32, 64);
+    if (g == 0) out[OFF_B1 + col] = db;
   }
 }
+
 
 // grad[p] = sum_w partial[w][p] (fixed order)
 __global__ void reduce_grad_kernel(const float *__restrict__ partial, int nwaves,
@@ -725,7 +781,17 @@ __global__ void reduce_grad_kernel(const float *__restrict__ partial, int nwaves
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= NPARAMS) return;
   float s = 0.0f;
-  for (int w = 0; w < nwaves; ++w) s += partial[static_cast<size_t>(w) * NPARAMS + p];
+  // sixteen reads in flight, added in order
+  constexpr int U = 16;
+  for (int w = 0; w < nwaves; w += U) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = partial[static_cast<size_t>(w + u < nwaves ? w + u : w) * NPARAMS + p];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (w + u < nwaves) s += v[u];
+  }
   grad[p] = s;
 }
 
@@ -792,6 +858,8 @@ __global__ void mfma_probe_kernel(float *out) {
 size_t lds_bytes_forward(int n) {
   return static_cast<size_t>(n >= kInPlaceMinN ? 1 : 2) * 16 * n * CH * 2 + 32 * CH * 2;
 }
+// h2, then h1 under the FP32 layer-3 activations
+size_t lds_bytes_forward_store(int n) { return static_cast<size_t>(3) * 16 * n * CH * 2; }
 size_t lds_bytes_backward(int n) { return static_cast<size_t>(3) * 16 * n * CH * 2; }
 
 } // namespace
@@ -868,6 +936,10 @@ int spined_cnn_forward_device(const spined_cnn *c, int n, uint64_t count, const 
     const unsigned blocks = static_cast<unsigned>((count + 15) / 16);
     if (!z_store && n >= spined::kInferMinN)
       spined::launch_infer(c->m, a, blocks, states, out_a, out_t, spined::stream());
+    else if (z_store && spined::lds_bytes_forward_store(n) <= (size_t(64) << 10))
+      hipLaunchKernelGGL(spined::cnn_forward_store_kernel, dim3(blocks),
+                         dim3(64 * spined::kFwdWaves), spined::lds_bytes_forward_store(n),
+                         spined::stream(), a, states, out_a, out_t, z_store);
     else
       hipLaunchKernelGGL(spined::cnn_forward_kernel, dim3(blocks), dim3(64),
                          spined::lds_bytes_forward(n), spined::stream(), a, states, out_a, out_t,
@@ -888,11 +960,11 @@ int spined_cnn_backward_device(spined_cnn *c, int n, uint64_t count, const uint6
     const unsigned blocks = static_cast<unsigned>((count + 15) / 16);
     DeviceBuffer<float> partial(static_cast<size_t>(blocks) * spined::NPARAMS);
     hipStream_t s = spined::stream();
-    hipLaunchKernelGGL(spined::cnn_backward_kernel, dim3(blocks), dim3(64),
+    hipLaunchKernelGGL(spined::cnn_backward_kernel, dim3(blocks), dim3(64 * spined::kBwdWaves),
                        spined::lds_bytes_backward(n), s, a, states, z_store, ga, gt, partial.ptr);
     SPINED_CHECK_LAUNCH();
     float *dst = grad_out ? grad_out : c->m.grad.ptr;
-    hipLaunchKernelGGL(spined::reduce_grad_kernel, dim3((spined::NPARAMS + 255) / 256), dim3(256),
+    hipLaunchKernelGGL(spined::reduce_grad_kernel, dim3((spined::NPARAMS + 63) / 64), dim3(64),
                        0, s, partial.ptr, static_cast<int>(blocks), dst);
     SPINED_CHECK_LAUNCH();
     SPINED_HIP(hipStreamSynchronize(s)); // `partial` is released at scope exit
