@@ -1056,18 +1056,15 @@ void launch_cached(const Operator &op, const Ctx &c, const GatherCache &gc, cons
 
 // Workgroup order of the cached kernels: each XCD a contiguous eighth of the
 // rows (xcd_block), or the dispatch order (consecutive waves on different
-// XCDs).  Ring orbits and plain sectors keep the targets of neighbouring
-// rows together, which an XCD's own L2 serves (D = 6.3e7 ring, FP64: 5.13 ms
-// contiguous, 5.44 in dispatch order; D = 5.2e6 without symmetries, FP32:
-// 123 against 161 us); with FP32 x of a ring the two are equal there and the
-// dispatch order is faster at D = 8.6e8 (85 against 89 ms).  Orbits of other
-// groups scatter them, and the XCDs then share the window's lines in the
-// Infinity Cache (6x6 square lattice, FP64: 4.52 ms in dispatch order, 4.75
-// contiguous; FP32: 3.60 against 3.88).
+// XCDs).  Neighbouring rows share gather targets, which an XCD's own L2 then
+// serves (contiguous against dispatch order, one FP64 vector: D = 6.3e7 ring
+// 4.99 and 5.26 ms, 8x4 torus, D = 9.4e6, 1.80 and 2.12, 5x7, D = 9.3e7, 15.7
+// and 18.6, 32-site pyrochlore with four vectors 0.46 and 0.56, 6x6 square
+// with its point group 4.44 and 4.42; without symmetries, D = 5.2e6, FP32, 123
+// and 161 us).  For FP32 x of a ring the dispatch order is faster at D = 8.6e8
+// (85 against 89 ms; 4.05 and 3.93 at 6.3e7).
 bool contiguous_rows(const Operator &op, bool f32) {
-  const auto &t = op.basis->tables;
-  if (t.nperm == 1) return true;
-  return t.ring_available && !f32;
+  return !(op.basis->tables.ring_available && f32);
 }
 
 // Low sites of the split row gather for a basis, or -1 where it does not
