@@ -1015,7 +1015,7 @@ int spined_debug_orbit(const ls_spin_basis *basis, int method, uint64_t count,
     if (method == 1 && !b.tables.ring_available)
       throw Error(LS_INVALID_ARGUMENT, "ring method unavailable for this group");
     auto ga = b.tables.generic_args(false);
-    if (method == 2) ga.torus_l1 = 0; // one program per element, no torus factorisation
+    if (method == 2) ga.torus_l1 = ga.key_orbit = 0; // one program per element, no torus factorisation
     const auto ra = b.tables.ring_args(false);
     for (uint64_t i = 0; i < count; ++i) {
       if (method == 3) { // the minimum alone (orbit_min_generic); no phase, count or validity

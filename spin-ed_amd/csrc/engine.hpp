@@ -70,9 +70,11 @@ struct OrbitTables {
   std::vector<uint32_t> h_point_elem;
   std::vector<int32_t> h_tp_phase;
   std::vector<uint64_t> h_row_lo, h_row_hi;
+  std::vector<uint32_t> h_row_key; // empty: l1 above kRowKeyMax
   DeviceBuffer<uint32_t> point_elem;
   DeviceBuffer<int32_t> tp_phase;
   DeviceBuffer<uint64_t> row_lo, row_hi;
+  DeviceBuffer<uint32_t> row_key;
   // sqrt(c / s) for stabiliser sizes c, s (divisors of |G|): ratio[i * nd + j]
   // with i = div_idx[c], j = div_idx[s]; nd = 0 when |G| is too large.
   int nd = 0;

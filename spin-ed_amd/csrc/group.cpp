@@ -129,6 +129,8 @@ GenericOrbitArgs OrbitTables::generic_args(bool device) const {
     a.tp_phase = device ? tp_phase.ptr : h_tp_phase.data();
     a.row_lo = device ? row_lo.ptr : h_row_lo.data();
     a.row_hi = device ? row_hi.ptr : h_row_hi.data();
+    a.key_orbit = h_row_key.empty() ? 0 : use_key_orbit(torus_l1, a.n_point);
+    a.row_key = h_row_key.empty() ? nullptr : device ? row_key.ptr : h_row_key.data();
   }
   return a;
 }
@@ -170,6 +172,7 @@ void detect_torus(const Group &g, int n, OrbitTables &t) {
   t.h_tp_phase.clear();
   t.h_row_lo.clear();
   t.h_row_hi.clear();
+  t.h_row_key.clear();
   if (g.n != n || n < 4 || t.ring_available) return;
   std::map<std::vector<uint8_t>, int> index;
   for (int e = 0; e < t.nperm; ++e) index.emplace(g.perms[e], e);
@@ -226,6 +229,21 @@ void detect_torus(const Group &g, int n, OrbitTables &t) {
       const uint64_t hi = ((1ull << l1) - 1) & ~lo; // row bits l1-dx .. l1-1
       t.h_row_lo.push_back(lo * rows);
       t.h_row_hi.push_back(hi * rows);
+    }
+    if (l1 <= kRowKeyMax) {
+      const uint32_t rm = (1u << l1) - 1u;
+      for (uint32_t v = 0; v <= rm; ++v) {
+        uint32_t key = rm, at = 0;
+        for (int b = 0; b < 16; ++b) {
+          const int dx = b & 7;
+          if (dx >= l1 || (b >= 8 && !t.has_flip)) continue;
+          const uint32_t r = ((v >> dx) | (v << (l1 - dx))) & rm;
+          const uint32_t z = b >= 8 ? r ^ rm : r;
+          if (z < key) key = z, at = 0;
+          if (z == key) at |= 1u << b;
+        }
+        t.h_row_key.push_back(key | at << 8);
+      }
     }
     return;
   }
@@ -347,6 +365,7 @@ void ensure_device(OrbitTables &t) {
   upload(t.tp_phase, t.h_tp_phase);
   upload(t.row_lo, t.h_row_lo);
   upload(t.row_hi, t.h_row_hi);
+  upload(t.row_key, t.h_row_key);
   upload(t.div_idx, t.h_div_idx);
   upload(t.ratio, t.h_ratio);
   t.on_device = true;

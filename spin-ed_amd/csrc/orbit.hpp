@@ -82,6 +82,12 @@ struct GenericOrbitArgs {
   const int32_t *__restrict__ tp_phase;
   const uint64_t *__restrict__ row_lo;
   const uint64_t *__restrict__ row_hi;
+  // row_key[v] (l1 <= kRowKeyMax; else null), for a row of l1 bits: the least
+  // value among its in-row rotations (and, with the flip, theirs
+  // complemented) in bits 0..7, the rotations dx that reach it plain in bits
+  // 8..15 and complemented in bits 16..23
+  const uint32_t *__restrict__ row_key;
+  int32_t key_orbit; // the orbit scans use row_key too
   int32_t torus_l1;
   int32_t torus_l2;
   int32_t n_point;
@@ -101,12 +107,145 @@ __host__ __device__ inline uint64_t apply_program(const GenericOrbitArgs &a, int
   return y;
 }
 
+// Row keys, for rows of up to eight bits.  The representative test takes them
+// wherever they are there: most candidates fail on their own top row, before
+// any image (half-filled 6x6 lattice with inversion and point group, 4.5e9
+// candidates: 106 -> 19 ms; 4x8 translations: 7.6 -> 4.4 for a whole build).
+// The orbit scans take them (key_orbit) for rows of six bits and more, and of
+// five where there are point elements: short rows tie often, and then the
+// images left cost more than the scan's rotations (first matvec, row keys
+// against scan: 6x6 62 and 97 ms, 8x4 8.5 and 9.7, 5x7 with reflections 50
+// and 64; 5x7 translations alone 106 and 96, 4x8 10.8 and 8.9, 2x16 13 and 8).
+constexpr int kRowKeyMax = 8;
+__host__ __device__ inline int use_key_orbit(int l1, int n_point) {
+  return l1 >= 6 || (l1 == 5 && n_point > 1) ? 1 : 0;
+}
+
+// Rows of the torus image y whose key equals the least of `key` and all of
+// y's row keys, which becomes `key` (bit r: row r; 0: no row reaches it).
+__host__ __device__ inline uint32_t torus_rows(const GenericOrbitArgs &a, uint64_t y,
+                                               uint32_t &key) {
+  const uint32_t rm = (1u << a.torus_l1) - 1u;
+  uint32_t rows = 0;
+  for (int r = 0; r < a.torus_l2; ++r) {
+    const uint32_t k = a.row_key[static_cast<uint32_t>(y) & rm] & 0xffu;
+    rows = k < key ? 0u : rows;
+    key = k < key ? k : key;
+    rows |= (k == key ? 1u : 0u) << r;
+    y >>= a.torus_l1;
+  }
+  return rows;
+}
+
+// Calls f(image, dx, dy, flipped) for the translations (and flips) of y that
+// put one of `rows` on top at its key: the only ones that can be the orbit's
+// least.  One loop over both the rows and their rotations, so a wave takes as
+// many turns as its longest lane has images, not as each row in turn would.
+// Stops when f returns false.
+template <class F>
+__host__ __device__ inline bool torus_candidates(const GenericOrbitArgs &a, uint64_t y,
+                                                 uint32_t rows, F &&f) {
+  const int l1 = a.torus_l1, l2 = a.torus_l2, n = a.n_sites;
+  const uint32_t rm = (1u << l1) - 1u;
+  uint32_t at = 0;
+  int dy = 0;
+  while (at | rows) {
+    if (!at) {
+      const int r = __builtin_ctz(rows);
+      rows &= rows - 1;
+      dy = r + 1 == l2 ? 0 : r + 1; // brings row r to the top
+      at = a.row_key[static_cast<uint32_t>(y >> (r * l1)) & rm] >> 8;
+    }
+    const int b = __builtin_ctz(at);
+    at &= at - 1;
+    const int dx = b & 7;
+    const uint64_t lo = a.row_lo[dx];
+    uint64_t z = (((y >> dx) & lo) | ((y << (l1 - dx)) & ~lo)) & a.site_mask;
+    const int k = dy * l1;
+    z = k == 0 ? z : (((z >> k) | (z << (n - k))) & a.site_mask);
+    if (!f(b >= 8 ? z ^ a.site_mask : z, dx, dy, b >= 8)) return false;
+  }
+  return true;
+}
+
+// orbit_torus by row keys: the least image starts with the least row key of
+// all images, so only the translations that put such a row on top (a few of
+// l1 l2, with the flip 2 l1 l2) are evaluated.  Same result.
+__host__ __device__ inline OrbitResult orbit_torus_key(const GenericOrbitArgs &a, uint64_t x) {
+  const uint64_t rx = reverse_n(x, a.n_sites);
+  uint64_t best = ~0ull;
+  int32_t ph = 0, cnt = 0;
+  bool ok = true;
+  uint32_t key = 0xffu;
+  for (int p = 0; p < a.n_point; ++p) {
+    const uint64_t y = apply_program(a, static_cast<int>(a.point_elem[p]), x, rx);
+    const int32_t *tph = a.tp_phase + p * a.torus_l1 * a.torus_l2;
+    torus_candidates(a, y, torus_rows(a, y, key), [&](uint64_t z, int dx, int dy, bool flipped) {
+      int32_t q = 0;
+      if (!a.trivial) {
+        q = tph[dy * a.torus_l1 + dx] + (flipped ? a.flip_phase : 0);
+        if (q >= a.L) q -= a.L;
+      }
+      // an image of a smaller key replaces every earlier one by itself
+      orbit_update(best, ph, cnt, ok, z, q);
+      return true;
+    });
+  }
+  return OrbitResult{best, ph, cnt, ok};
+}
+
+__host__ __device__ inline uint64_t orbit_min_torus_key(const GenericOrbitArgs &a, uint64_t x) {
+  const uint64_t rx = reverse_n(x, a.n_sites);
+  uint64_t best = ~0ull;
+  uint32_t key = 0xffu;
+  for (int p = 0; p < a.n_point; ++p) {
+    const uint64_t y = apply_program(a, static_cast<int>(a.point_elem[p]), x, rx);
+    torus_candidates(a, y, torus_rows(a, y, key), [&](uint64_t z, int, int, bool) {
+      best = z < best ? z : best;
+      return true;
+    });
+  }
+  return best;
+}
+
+// rep_test_generic by row keys: x fails as soon as some row's key is below
+// x's own top row.
+__host__ __device__ inline uint32_t rep_test_torus_key(const GenericOrbitArgs &a, uint64_t x) {
+  const uint32_t top = static_cast<uint32_t>(x >> (a.n_sites - a.torus_l1));
+  if ((a.row_key[top] & 0xffu) < top) return 0;
+  const uint64_t rx = reverse_n(x, a.n_sites);
+  uint32_t cnt = 0;
+  for (int p = 0; p < a.n_point; ++p) {
+    const uint64_t y = apply_program(a, static_cast<int>(a.point_elem[p]), x, rx);
+    uint32_t key = top;
+    const uint32_t rows = torus_rows(a, y, key);
+    if (key < top) return 0;
+    const int32_t *tph = a.tp_phase + p * a.torus_l1 * a.torus_l2;
+    if (!torus_candidates(a, y, rows, [&](uint64_t z, int dx, int dy, bool flipped) {
+          if (z < x) return false;
+          if (z == x) {
+            int32_t q = 0;
+            if (!a.trivial) {
+              q = tph[dy * a.torus_l1 + dx] + (flipped ? a.flip_phase : 0);
+              if (q >= a.L) q -= a.L;
+            }
+            if (q != 0) return false;
+            ++cnt;
+          }
+          return true;
+        }))
+      return 0;
+  }
+  return cnt;
+}
+
 // Orbit over the torus factorisation: the point element's program once,
 // then the l1 in-row rotations (two masked shifts each) and, for each, the
 // l2 row rotations (one rotation of the word by l1 sites each).  Same
 // (rep, count, valid) as the scan over every element; the phase is that of
 // an element reaching rep (all of them carry it when valid).
 __host__ __device__ inline OrbitResult orbit_torus(const GenericOrbitArgs &a, uint64_t x) {
+  if (a.key_orbit) return orbit_torus_key(a, x);
   const uint64_t rx = reverse_n(x, a.n_sites);
   const int l1 = a.torus_l1, l2 = a.torus_l2, n = a.n_sites;
   const uint64_t mask = a.site_mask;
@@ -166,6 +305,7 @@ __host__ __device__ inline OrbitResult orbit_generic(const GenericOrbitArgs &a, 
 // entry of the representative): the scans of orbit_torus / orbit_generic
 // without the count and phase bookkeeping.  Same rep as orbit_generic.
 __host__ __device__ inline uint64_t orbit_min_generic(const GenericOrbitArgs &a, uint64_t x) {
+  if (a.key_orbit) return orbit_min_torus_key(a, x);
   const uint64_t rx = reverse_n(x, a.n_sites);
   const uint64_t mask = a.site_mask;
   uint64_t best = ~0ull;
@@ -205,6 +345,7 @@ __host__ __device__ inline uint64_t orbit_min_generic(const GenericOrbitArgs &a,
 // else 0.
 // rep_test_generic over the torus factorisation (same result).
 __host__ __device__ inline uint32_t rep_test_torus(const GenericOrbitArgs &a, uint64_t x) {
+  if (a.row_key) return rep_test_torus_key(a, x);
   const uint64_t rx = reverse_n(x, a.n_sites);
   const int l1 = a.torus_l1, l2 = a.torus_l2, n = a.n_sites;
   const uint64_t mask = a.site_mask;
