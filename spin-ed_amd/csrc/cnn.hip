@@ -633,12 +633,14 @@ __device__ inline void weight_grad(const __bf16 *dz, const __bf16 *h, const uint
   }
 }
 
-// Backward pass of 16 samples: kBwdWaves waves, one per tap of the weight
-// gradients; the data gradients and activations are split by position.  One
-// wave ran all of it in turn on half of the chip (2,048 samples of 30 sites: 151
-// us; now 69).
+// Backward pass of 16 samples: the first KW waves form the weight gradients,
+// one tap each, while the others form the data gradient that the next layer
+// needs; activations are split by position over all.  Bound: the latency of
+// each wave's chain of LDS reads, products and activations, on the half of the
+// chip that 2,048 samples fill.  2,048 samples of 30 sites: one wave for all of
+// it 151 us, five waves that do both in turn 70, ten 61.
 // Every sum is formed by one wave in the order of the one-wave kernel.
-constexpr int kBwdWaves = KW;
+constexpr int kBwdWaves = 2 * KW;
 __global__ void __launch_bounds__(64 * kBwdWaves)
     cnn_backward_kernel(CnnArgs c, const uint64_t *__restrict__ states,
                         const float *__restrict__ z_store, const float *__restrict__ ga,
@@ -734,7 +736,7 @@ __global__ void __launch_bounds__(64 * kBwdWaves)
   auto data_grad = [&](const __bf16 *d, int off_w, const float *z, __bf16 *dst) {
     bf16x8 a[3];
     load_conv_weights(P + off_w, true, a);
-    for (int pos = wv; pos < n; pos += kBwdWaves) {
+    for (int pos = wv - KW; pos < n; pos += kBwdWaves - KW) {
       floatx4 acc = conv_at(a, d, n, pos);
       floatx4 zz = load4_f32(z, n, pos);
 #pragma unroll
@@ -743,11 +745,13 @@ __global__ void __launch_bounds__(64 * kBwdWaves)
     }
   };
 
-  // layer 3 weight gradient (dz = bufA, h = bufB)
-  wgrad(bufA, bufB, OFF_W3, OFF_B3);
+  // layer 3 weight gradient (dz = bufA, h = bufB); d2 -> bufC
+  if (wv < KW)
+    wgrad(bufA, bufB, OFF_W3, OFF_B3);
+  else
+    data_grad(bufA, OFF_W3, z2, bufC);
   __syncthreads();
-  // d2 -> bufC; h1 = gelu(z1) -> bufB
-  data_grad(bufA, OFF_W3, z2, bufC);
+  // h1 = gelu(z1) -> bufB; bufA is free
   for (int pos = wv; pos < n; pos += kBwdWaves) {
     floatx4 z = load4_f32(z1, n, pos), h;
 #pragma unroll
@@ -756,8 +760,10 @@ __global__ void __launch_bounds__(64 * kBwdWaves)
   }
   __syncthreads();
   // layer 2 weight gradient (dz = bufC, h = bufB); d1 -> bufA
-  wgrad(bufC, bufB, OFF_W2, OFF_B2);
-  data_grad(bufC, OFF_W2, z1, bufA);
+  if (wv < KW)
+    wgrad(bufC, bufB, OFF_W2, OFF_B2);
+  else
+    data_grad(bufC, OFF_W2, z1, bufA);
   __syncthreads();
   // layer 1 weight gradient (dz = bufA, input spins): one product for all taps
   if (wv == 0) {
