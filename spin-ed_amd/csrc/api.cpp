@@ -220,14 +220,14 @@ size_t elem_size(int dtype) {
 
 // Locks the operator's basis for device work: builds are serialised with
 // matvecs, and device tables are uploaded on first use.
-Operator &prepare_operator(const ls_operator *op) {
+Operator &prepare_operator(const ls_operator *op, bool repeated = false) {
   if (!op || !op->p) throw Error(LS_INVALID_ARGUMENT, "operator is NULL");
   Operator &o = *op->p;
   Basis &b = *o.basis;
   require_built(b);
   ensure_basis_device(b);
   ensure_device(o.tables);
-  ensure_schedule(o);
+  ensure_schedule(o, repeated);
   ++o.cache->calls;
   return o;
 }
@@ -556,7 +556,7 @@ int spined_eigsh(const ls_operator *op, int dtype, uint64_t k, double tol,
                  double *rnorms, spined_monitor_fn monitor, void *monitor_ctx) {
   int status = LS_SUCCESS;
   const int g = guarded([&] {
-    Operator &o = prepare_operator(op);
+    Operator &o = prepare_operator(op, true);
     if (!evals) throw Error(LS_INVALID_ARGUMENT, "evals is NULL");
     spined_eigsh_options d;
     spined_eigsh_options_init(&d);

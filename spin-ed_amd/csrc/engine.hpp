@@ -317,7 +317,8 @@ struct Operator {
 
 constexpr int kScheduleTile = 4096;
 constexpr int kRowsPerWaveMax = 64; // one lane per row
-void ensure_schedule(Operator &op); // matvec.hip
+// matvec.hip; repeated: more matvecs are known to follow
+void ensure_schedule(Operator &op, bool repeated = false);
 // Drops the operator's gather cache (the schedule or the basis changed).
 void drop_gather_cache(Operator &op);  // matvec.hip
 // Frees the gather caches on a device (a device allocation failed).

@@ -849,11 +849,23 @@ constexpr uint64_t kCacheReserve = uint64_t(4) << 30;
 constexpr uint64_t kCacheMinRows = uint64_t(1) << 20;
 constexpr uint64_t kCacheTinyRows = 64;
 constexpr double kCacheFirstWork = 2e9;
-constexpr uint64_t kCacheMaxClasses = 65536; // 16-bit class numbers
 
 int unit_count(const OperatorTables &t) {
   return t.bonds ? static_cast<int>(t.h_bond_sites.size()) : t.ntemplates;
 }
+
+// Whether an automatic cache of the operator is due at its `calls`-th use.
+bool cache_due(const Operator &op, int calls) {
+  const Basis &b = *op.basis;
+  if (b.D >= kCacheMinRows) return true;
+  if (b.D <= kCacheTinyRows) return false;
+  const double orbit = op.orbit_method() == 1 ? 64.0 : 2.0 * b.tables.orbit_cost;
+  return calls >= 2 ||
+         static_cast<double>(b.D) * unit_count(op.tables) * orbit >= kCacheFirstWork;
+}
+
+// 16-bit class numbers
+constexpr uint64_t kCacheMaxClasses = 65536;
 
 // Coefficient classes: every distinct unit coefficient times every phase
 // that an orbit can return, with the products of matvec_complex_kernel (and,
@@ -954,12 +966,8 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
     explicit Building(std::atomic<bool> &x) : f(x) { f.store(true); }
     ~Building() { f.store(false); }
   } building(gc.building);
-  if (gc.request < 0 && b.D < kCacheMinRows) {
-    if (b.D <= kCacheTinyRows) return false;
-    const double orbit = METHOD == 1 ? 64.0 : 2.0 * b.tables.orbit_cost;
-    if (!repeated && static_cast<double>(b.D) * units * orbit < kCacheFirstWork && gc.calls.load() < 2)
-      return false;
-  }
+  if (gc.request < 0 && !(repeated && b.D > kCacheTinyRows) && !cache_due(op, gc.calls.load()))
+    return false;
   const uint64_t waves = (b.D + kRowBlock - 1) / kRowBlock;
   const unsigned g = static_cast<unsigned>(waves);
   if (!gc.counted) {
@@ -1413,7 +1421,7 @@ void launch_rows_to_cols(VecType t, const void *yr, uint64_t D, int K, void *y, 
 
 int block_chunk(uint64_t remaining) { return remaining >= 8 ? 8 : remaining >= 4 ? 4 : remaining >= 2 ? 2 : 1; }
 
-void ensure_schedule(Operator &op) {
+void ensure_schedule(Operator &op, bool repeated) {
   std::lock_guard<std::mutex> lk(op.mu);
   const Basis &b = *op.basis;
   // automatic: bases of at least one tile
@@ -1426,8 +1434,21 @@ void ensure_schedule(Operator &op) {
     return;
   }
   if (op.schedule_built) return;
-  drop_gather_cache(op);
   hipStream_t s = stream();
+  // Complex operators and those of many templates use it through the gather
+  // cache alone: an automatic schedule waits until that is due (a first
+  // complex matvec of 9,252 rows took 328 us with it, 264 without).
+  const int units = unit_count(op.tables);
+  if (op.schedule_request < 0 && (!op.tables.is_real || units > (op.tables.bonds ? 128 : 256))) {
+    GatherCache &gc = *op.cache;
+    std::lock_guard<std::mutex> cache_lock(gc.mu);
+    if (gc.built || gc.request == 0) return;
+    if (gc.request < 0 && !repeated && !cache_due(op, gc.calls.load() + 1)) return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    SPINED_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone) return;
+  }
+  drop_gather_cache(op);
   op.sched.allocate(b.D);
   const Ctx c = make_ctx(op, nullptr, nullptr);
   const unsigned tiles = static_cast<unsigned>((b.D + kScheduleTile - 1) / kScheduleTile);
