@@ -1437,7 +1437,7 @@ void ensure_schedule(Operator &op, bool repeated) {
   hipStream_t s = stream();
   // Complex operators and those of many templates use it through the gather
   // cache alone: an automatic schedule waits until that is due (a first
-  // complex matvec of 9,252 rows took 328 us with it, 264 without).
+  // complex matvec of 9,252 rows took 328 us with it, 309 without).
   const int units = unit_count(op.tables);
   if (op.schedule_request < 0 && (!op.tables.is_real || units > (op.tables.bonds ? 128 : 256))) {
     GatherCache &gc = *op.cache;
