@@ -338,6 +338,10 @@ int spined_debug_ring_available(const ls_spin_basis *basis);
  * x, and each element is a translation after one of a few point elements);
  * 0 x 0 when the orbit runs one program per element. */
 int spined_debug_torus_shape(const ls_spin_basis *basis, int32_t *l1, int32_t *l2);
+/* Eigenpairs of the symmetric m x m matrix `a` (row-major, host memory, 1 <= m
+ * <= 64) by the eigensolvers' projected-matrix kernel: evals ascending, vecs[i *
+ * m + j] component j of eigenvector i. */
+int spined_debug_eigh(int32_t m, const double *a, double *evals, double *vecs);
 /* Plain device copy of `bytes` (multiple of 16): the calibration kernel for
  * HBM byte counters in profiles. */
 int spined_debug_copy_device(void *dst, const void *src, uint64_t bytes);

@@ -1057,6 +1057,14 @@ int spined_debug_orbit_hop(const ls_spin_basis *basis, uint64_t count, const uin
   });
 }
 
+int spined_debug_eigh(int32_t m, const double *a, double *evals, double *vecs) {
+  return guarded([&] {
+    if (m < 1 || m > 64 || !a || !evals || !vecs)
+      throw Error(LS_INVALID_ARGUMENT, "matrix size must be 1 to 64");
+    projected_eigh(m, a, evals, vecs);
+  });
+}
+
 int spined_debug_copy_device(void *dst, const void *src, uint64_t bytes) {
   return guarded([&] {
     if (!dst || !src || bytes % 16) throw Error(LS_INVALID_ARGUMENT, "bytes must be a multiple of 16");

@@ -375,6 +375,8 @@ int block_chunk(uint64_t remaining);
 uint64_t count_offdiag_device(const Operator &op);
 
 // ---- eigensolver (solver.hip) ---------------------------------------------
+// Test hook: eigenpairs of a host matrix by the projected-matrix kernel.
+void projected_eigh(int m, const double *a, double *evals, double *vecs); // solver.hip
 int eigsh(Operator &op, int dtype, uint64_t k, double tol, const spined_eigsh_options &opts,
           double *evals, void *evecs, uint64_t ld, double *rnorms, spined_monitor_fn monitor,
           void *ctx);

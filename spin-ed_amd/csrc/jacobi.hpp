@@ -29,19 +29,22 @@ __device__ inline void jacobi_rotation(double app, double aqq, double apq, doubl
 // Bound: the latency of one round's chain -- the rotation's two divisions and
 // two square roots, LDS, barriers -- about m - 1 rounds a sweep and 7 sweeps.
 // The 2 x 2 blocks A[pair k][pair l] are independent, so after the rotations
-// one step updates columns and rows together (k <= l; the mirror image is
-// copied) and V with them; the closing sort and copy run on all threads (one
-// thread took a third of the call).  Rotations by every block's thread
-// itself, without the barrier between, were slower (223 us against 177 for
-// three steps a round, m <= 24): the divisions then compete for issue.
+// one step updates columns and rows together and V with them.  Every ordered
+// pair (k, l) is computed from its own four entries, columns first, then rows:
+// the rounding of a pass over all columns followed by one over all rows.  (The
+// mirror image of a block has another rounding, and the sign of an eigenvector
+// of the block solver hangs on the last bit.)  Up to m = 32 that is one block a
+// thread.  The closing sort and copy run on all threads (one thread took a third
+// of the call).  Rotations by every block's thread itself, without the barrier
+// between, were slower (223 us against 177 for three steps a round, m <= 24): the
+// divisions then compete for issue.
 template <int MAXM = kJacobiMax>
 __device__ inline void jacobi_eigh_device(const double *__restrict__ T, int ldt, int m,
                                           double *__restrict__ evals, double *__restrict__ S,
                                           int max_sweeps) {
   static_assert(MAXM % 2 == 0 && MAXM <= kJacobiMax, "even size up to kJacobiMax");
   constexpr int kHalf = MAXM / 2;
-  // blocks k <= l only (A stays symmetric)
-  constexpr int kBlocks = (kHalf * (kHalf + 1) / 2 + kJacobiThreads - 1) / kJacobiThreads;
+  constexpr int kBlocks = (kHalf * kHalf + kJacobiThreads - 1) / kJacobiThreads;
   __shared__ double A[MAXM][MAXM + 1];
   __shared__ double V[MAXM][MAXM + 1];
   __shared__ double cs[kHalf], sn[kHalf];
@@ -49,7 +52,6 @@ __device__ inline void jacobi_eigh_device(const double *__restrict__ T, int ldt,
   const int tid = threadIdx.x;
   const int mp = m + (m & 1);
   const int half = mp / 2;
-  const int nblk = half * (half + 1) / 2;
   for (int e = tid; e < mp * mp; e += kJacobiThreads) {
     const int i = e / mp, j = e % mp;
     double a = 0.0;
@@ -57,22 +59,13 @@ __device__ inline void jacobi_eigh_device(const double *__restrict__ T, int ldt,
     A[i][j] = a;
     V[i][j] = i == j ? 1.0 : 0.0;
   }
-  // the pairs (k, l) of this thread's blocks, k <= l
+  // the pairs (k, l) of this thread's blocks
   int bk[kBlocks], bl[kBlocks];
 #pragma unroll
   for (int z = 0; z < kBlocks; ++z) {
-    int e = tid + z * kJacobiThreads;
-    bk[z] = -1;
-    bl[z] = 0;
-    if (e < nblk) {
-      int k = 0;
-      while (e >= half - k) {
-        e -= half - k;
-        ++k;
-      }
-      bk[z] = k;
-      bl[z] = k + e;
-    }
+    const int e = tid + z * kJacobiThreads;
+    bk[z] = e < half * half ? e / half : -1;
+    bl[z] = e % half;
   }
   __syncthreads();
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
@@ -137,12 +130,6 @@ __device__ inline void jacobi_eigh_device(const double *__restrict__ T, int ldt,
         A[p][t] = w1;
         A[q][r] = w2;
         A[q][t] = w3;
-        if (bk[z] != bl[z]) {
-          A[r][p] = w0;
-          A[t][p] = w1;
-          A[r][q] = w2;
-          A[t][q] = w3;
-        }
       }
       // V <- V J (columns p, q)
       for (int e = tid; e < half * mp; e += kJacobiThreads) {
@@ -158,16 +145,36 @@ __device__ inline void jacobi_eigh_device(const double *__restrict__ T, int ldt,
     }
   }
   __syncthreads();
-  // ascending order of the m real eigenpairs (the padding index is dropped):
-  // a pair's place is the number of smaller ones, ties by index
+  // ascending order of the m real eigenpairs (the padding index is dropped): a
+  // pair's place is the number of smaller ones; equal or unordered values take
+  // the order that a selection sort with exchanges leaves them in
   __shared__ int order[MAXM];
-  for (int i = tid; i < m; i += kJacobiThreads) order[i] = i; // stays valid if a value is NaN
+  __shared__ int serial;
+  if (tid == 0) serial = 0;
   __syncthreads();
   for (int i = tid; i < m; i += kJacobiThreads) {
     const double a = A[i][i];
     int at = 0;
-    for (int j = 0; j < m; ++j) at += A[j][j] < a || (A[j][j] == a && j < i) ? 1 : 0;
+    bool tie = false;
+    for (int j = 0; j < m; ++j) {
+      const double b = A[j][j];
+      at += b < a ? 1 : 0;
+      tie = tie || (j != i && !(b < a) && !(a < b));
+    }
     order[at] = i;
+    if (tie) serial = 1;
+  }
+  __syncthreads();
+  if (serial && tid == 0) {
+    for (int i = 0; i < m; ++i) order[i] = i;
+    for (int i = 0; i < m; ++i) {
+      int best = i;
+      for (int j = i + 1; j < m; ++j)
+        if (A[order[j]][order[j]] < A[order[best]][order[best]]) best = j;
+      const int t = order[i];
+      order[i] = order[best];
+      order[best] = t;
+    }
   }
   __syncthreads();
   for (int i = tid; i < m; i += kJacobiThreads) evals[i] = A[order[i]][order[i]];

@@ -1272,6 +1272,18 @@ void dense_small_eigsh(Operator &op, uint64_t n, uint64_t k, int dtype, double *
   }
 }
 
+void projected_eigh(int m, const double *a, double *evals, double *vecs) {
+  hipStream_t s = stream();
+  const size_t mm = static_cast<size_t>(m) * m;
+  DeviceBuffer<double> T(mm), th(m), S(mm);
+  copy_in(T.ptr, a, 8 * mm);
+  jacobi_eigh_kernel<<<1, kJacobiThreads, 0, s>>>(T.ptr, m, m, th.ptr, S.ptr, 40);
+  SPINED_CHECK_LAUNCH();
+  SPINED_HIP(hipMemcpyAsync(evals, th.ptr, 8 * m, hipMemcpyDeviceToHost, s));
+  SPINED_HIP(hipMemcpyAsync(vecs, S.ptr, 8 * mm, hipMemcpyDeviceToHost, s));
+  SPINED_HIP(hipStreamSynchronize(s));
+}
+
 int eigsh(Operator &op, int dtype, uint64_t k, double tol, const spined_eigsh_options &opts_in,
           double *evals, void *evecs, uint64_t ld, double *rnorms, spined_monitor_fn monitor,
           void *ctx) {

@@ -479,6 +479,18 @@ def debug_orbit_hop(basis: SpinBasis, states, sites):
     return reps, ph, cnt, val.astype(bool)
 
 
+def debug_eigh(a):
+    """Eigenvalues and eigenvectors (rows) of a symmetric matrix of up to 64
+    rows by the eigensolvers' projected-matrix kernel (test hook)."""
+    a = np.ascontiguousarray(a, dtype=np.float64)
+    m = len(a)
+    if a.shape != (m, m):
+        raise ValueError("square matrix expected")
+    evals, vecs = np.empty(m), np.empty((m, m))
+    check_status(_lib.load().spined_debug_eigh(m, a.ctypes.data, evals.ctypes.data, vecs.ctypes.data))
+    return evals, vecs
+
+
 def ring_available(basis: SpinBasis) -> bool:
     return bool(_lib.load().spined_debug_ring_available(basis.ptr))
 
