@@ -220,14 +220,14 @@ size_t elem_size(int dtype) {
 
 // Locks the operator's basis for device work: builds are serialised with
 // matvecs, and device tables are uploaded on first use.
-Operator &prepare_operator(const ls_operator *op, bool repeated = false) {
+Operator &prepare_operator(const ls_operator *op) {
   if (!op || !op->p) throw Error(LS_INVALID_ARGUMENT, "operator is NULL");
   Operator &o = *op->p;
   Basis &b = *o.basis;
   require_built(b);
   ensure_basis_device(b);
   ensure_device(o.tables);
-  ensure_schedule(o, repeated);
+  ensure_schedule(o);
   ++o.cache->calls;
   return o;
 }
@@ -556,7 +556,7 @@ int spined_eigsh(const ls_operator *op, int dtype, uint64_t k, double tol,
                  double *rnorms, spined_monitor_fn monitor, void *monitor_ctx) {
   int status = LS_SUCCESS;
   const int g = guarded([&] {
-    Operator &o = prepare_operator(op, true);
+    Operator &o = prepare_operator(op);
     if (!evals) throw Error(LS_INVALID_ARGUMENT, "evals is NULL");
     spined_eigsh_options d;
     spined_eigsh_options_init(&d);
@@ -921,7 +921,11 @@ int spined_operator_set_schedule(ls_operator *op, int mode) {
 }
 
 int spined_operator_get_schedule(const ls_operator *op) {
-  return op ? (op->p->schedule_built ? 1 : 0) : -1;
+  if (!op) return -1;
+  if (op->p->schedule_built) return 1;
+  GatherCache &gc = *op->p->cache;
+  std::lock_guard<std::mutex> lk(gc.mu);
+  return gc.own_sched.ptr ? 1 : 0;
 }
 
 int spined_operator_set_rows_per_wave(ls_operator *op, int rows) {

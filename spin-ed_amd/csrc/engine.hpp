@@ -264,6 +264,12 @@ struct GatherCache {
   uint32_t imask = 0, cmask = 0;
   bool in_entry = true;   // classes fit in the entries
   double one[2] = {0, 0}; // class 0
+  // Slot order that woff and the entries follow, fixed when they are counted:
+  // the operator's row schedule, own_sched, or none.  The cached kernels take
+  // it from here, so that a call which prepared itself before the cache was
+  // built, on another thread, reads the cache in the order it was filled in.
+  const uint16_t *sched = nullptr;
+  DeviceBuffer<uint16_t> own_sched;
   DeviceBuffer<uint64_t> woff;
   DeviceBuffer<double> cls;        // nclass x (re, im)
   DeviceBuffer<uint16_t> unit_cls; // coefficient class of each unit
@@ -282,6 +288,8 @@ struct GatherCache {
     release_entries();
     counted = false;
     total = 0;
+    sched = nullptr;
+    own_sched.release();
     woff.release();
     cls.release();
     unit_cls.release();
@@ -299,7 +307,9 @@ struct Operator {
   // Row schedule of the matvec kernels: within every tile of
   // kScheduleTile consecutive rows, the rows ordered by their number of
   // active off-diagonal templates, so a wave's lanes carry equal work.
-  // sched[i] = offset within the tile of the row processed at slot i.
+  // sched[i] = offset within the tile of the row processed at slot i.  Operators
+  // whose matrix-free kernels do not use it have none here unless it was asked
+  // for: their gather cache makes its own.
   int schedule_request = -1; // -1 automatic, 0 off, 1 on
   // Lanes per row of the matrix-free real matvec of exchange-bond
   // operators: 1 (kRowsPerWaveMax rows per wave), 2 or 4; the sums do not
@@ -317,8 +327,7 @@ struct Operator {
 
 constexpr int kScheduleTile = 4096;
 constexpr int kRowsPerWaveMax = 64; // one lane per row
-// matvec.hip; repeated: more matvecs are known to follow
-void ensure_schedule(Operator &op, bool repeated = false);
+void ensure_schedule(Operator &op); // matvec.hip
 // Drops the operator's gather cache (the schedule or the basis changed).
 void drop_gather_cache(Operator &op);  // matvec.hip
 // Frees the gather caches on a device (a device allocation failed).

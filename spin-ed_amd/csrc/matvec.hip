@@ -929,6 +929,24 @@ bool cache_classes(const Operator &op, GatherCache &gc, hipStream_t s) {
   return true;
 }
 
+// Whether the row schedule serves the operator's gather cache alone: the
+// matrix-free kernels of complex operators and of those of many templates take
+// the rows in order.
+bool schedule_of_cache(const Operator &op) {
+  const auto &t = op.tables;
+  return !t.is_real || unit_count(t) > (t.bonds ? 128 : 256);
+}
+
+void launch_schedule(const Operator &op, const Ctx &c, uint16_t *sched, hipStream_t s) {
+  const Basis &b = *op.basis;
+  const unsigned tiles = static_cast<unsigned>((b.D + kScheduleTile - 1) / kScheduleTile);
+  if (c.bonds)
+    schedule_kernel<true><<<tiles, kSchedBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, sched);
+  else
+    schedule_kernel<false><<<tiles, kSchedBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, sched);
+  SPINED_CHECK_LAUNCH();
+}
+
 template <int METHOD, class F> void with_fill(const Ctx &c, F &&f) {
   const int units = c.bonds ? c.bd.nbonds : c.o.ntemplates;
   if (c.bonds && units <= 64)
@@ -976,11 +994,18 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
         throw Error(LS_NOT_IMPLEMENTED, "gather cache: too many distinct coefficients");
       return false;
     }
+    gc.sched = c.sched;
+    if (!gc.sched && schedule_of_cache(op) && op.schedule_request < 0 &&
+        b.D >= static_cast<uint64_t>(kScheduleTile)) {
+      gc.own_sched.allocate(b.D);
+      launch_schedule(op, c, gc.own_sched.ptr, s);
+      gc.sched = gc.own_sched.ptr;
+    }
     DeviceBuffer<uint32_t> wt(waves);
     if (c.bonds)
-      cache_count_kernel<true><<<g, kRowBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, c.sched, wt.ptr);
+      cache_count_kernel<true><<<g, kRowBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, gc.sched, wt.ptr);
     else
-      cache_count_kernel<false><<<g, kRowBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, c.sched,
+      cache_count_kernel<false><<<g, kRowBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, gc.sched,
                                                         wt.ptr);
     SPINED_CHECK_LAUNCH();
     gc.woff.allocate(waves + 1);
@@ -1019,7 +1044,7 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
   with_fill<METHOD>(c, [&](auto nw, auto bonds) {
     auto fill = [&](auto many) {
       cache_fill_kernel<METHOD, decltype(nw)::value, decltype(bonds)::value, decltype(many)::value>
-          <<<g, kRowBlock, 0, s>>>(c.o, c.bd, c.ga, c.ra, c.ix, c.stab, c.D, c.sched, gc.woff.ptr,
+          <<<g, kRowBlock, 0, s>>>(c.o, c.bd, c.ga, c.ra, c.ix, c.stab, c.D, gc.sched, gc.woff.ptr,
                                    gc.unit_cls.ptr, gc.phases, gc.shift,
                                    op.tables.is_real ? 0 : 1, gc.entries.ptr,
                                    gc.in_entry ? nullptr : gc.aux.ptr, gc.diag.ptr, gc.cnt.ptr);
@@ -1048,10 +1073,10 @@ void launch_cached(const Operator &op, const Ctx &c, const GatherCache &gc, cons
   auto go = [&](auto cm) {
     if (stream_entries)
       matvec_cached_kernel<R, decltype(cm)::value, true><<<g, kRowBlock, 0, s>>>(
-          ca, c.rt, c.stab, c.D, xp, yp, c.sched, contiguous ? 1 : 0, cdiag, one);
+          ca, c.rt, c.stab, c.D, xp, yp, gc.sched, contiguous ? 1 : 0, cdiag, one);
     else
       matvec_cached_kernel<R, decltype(cm)::value, false><<<g, kRowBlock, 0, s>>>(
-          ca, c.rt, c.stab, c.D, xp, yp, c.sched, contiguous ? 1 : 0, cdiag, one);
+          ca, c.rt, c.stab, c.D, xp, yp, gc.sched, contiguous ? 1 : 0, cdiag, one);
   };
   if (gc.nclass == 1)
     go(std::integral_constant<int, 0>{});
@@ -1421,7 +1446,7 @@ void launch_rows_to_cols(VecType t, const void *yr, uint64_t D, int K, void *y, 
 
 int block_chunk(uint64_t remaining) { return remaining >= 8 ? 8 : remaining >= 4 ? 4 : remaining >= 2 ? 2 : 1; }
 
-void ensure_schedule(Operator &op, bool repeated) {
+void ensure_schedule(Operator &op) {
   std::lock_guard<std::mutex> lk(op.mu);
   const Basis &b = *op.basis;
   // automatic: bases of at least one tile
@@ -1434,29 +1459,13 @@ void ensure_schedule(Operator &op, bool repeated) {
     return;
   }
   if (op.schedule_built) return;
+  // An automatic schedule that the cache alone would use comes with it (a first
+  // complex matvec of 9,252 rows took 328 us with a schedule, 309 without).
+  if (op.schedule_request < 0 && schedule_of_cache(op)) return;
   hipStream_t s = stream();
-  // Complex operators and those of many templates use it through the gather
-  // cache alone: an automatic schedule waits until that is due (a first
-  // complex matvec of 9,252 rows took 328 us with it, 309 without).
-  const int units = unit_count(op.tables);
-  if (op.schedule_request < 0 && (!op.tables.is_real || units > (op.tables.bonds ? 128 : 256))) {
-    GatherCache &gc = *op.cache;
-    std::lock_guard<std::mutex> cache_lock(gc.mu);
-    if (gc.built || gc.request == 0) return;
-    if (gc.request < 0 && !repeated && !cache_due(op, gc.calls.load() + 1)) return;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    SPINED_HIP(hipStreamIsCapturing(s, &cap));
-    if (cap != hipStreamCaptureStatusNone) return;
-  }
   drop_gather_cache(op);
   op.sched.allocate(b.D);
-  const Ctx c = make_ctx(op, nullptr, nullptr);
-  const unsigned tiles = static_cast<unsigned>((b.D + kScheduleTile - 1) / kScheduleTile);
-  if (c.bonds)
-    schedule_kernel<true><<<tiles, kSchedBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
-  else
-    schedule_kernel<false><<<tiles, kSchedBlock, 0, s>>>(c.o, c.bd, b.reps.ptr, b.D, op.sched.ptr);
-  SPINED_CHECK_LAUNCH();
+  launch_schedule(op, make_ctx(op, nullptr, nullptr), op.sched.ptr, s);
   SPINED_HIP(hipStreamSynchronize(s));
   op.schedule_built = true;
 }
