@@ -206,7 +206,8 @@ int spined_operator_get_rows_per_wave(const ls_operator *op);
  * matrix-free matvec is long, at the second call or at a solve otherwise;
  * not where the states split into halves that need no entries;
  * given back whenever a device allocation of the library needs the memory),
- * 0 off, 1 on (built at the next matvec; an error if it does not fit).  get:
+ * 0 off (the orbit-and-index kernels, also where the states split into
+ * halves), 1 on (built at the next matvec; an error if it does not fit).  get:
  * 1 while a cache is built.  Changing the row schedule drops the cache. */
 int spined_operator_set_gather_cache(ls_operator *op, int mode);
 int spined_operator_get_gather_cache(const ls_operator *op);
@@ -340,6 +341,9 @@ int spined_debug_ring_available(const ls_spin_basis *basis);
  * x, and each element is a translation after one of a few point elements);
  * 0 x 0 when the orbit runs one program per element. */
 int spined_debug_torus_shape(const ls_spin_basis *basis, int32_t *l1, int32_t *l2);
+/* Kernels that the operator's last matvec ran: 0 orbits and index, 1 gather
+ * cache, 2 split row gather (halves of the state); -1: none yet. */
+int spined_debug_matvec_path(const ls_operator *op);
 /* Eigenpairs of the symmetric m x m matrix `a` (row-major, host memory, 1 <= m
  * <= 64) by the eigensolvers' projected-matrix kernel: evals ascending, vecs[i *
  * m + j] component j of eigenvector i. */

@@ -801,8 +801,9 @@ int spined_operator_autotune(ls_operator *op, int32_t repeats, spined_autotune_r
       }
       ensure_schedule(o);
     };
-    // the tuner times the orbit-and-index kernels: the gather cache is off
-    // while it runs, and its request is restored afterwards
+    // the tuner times the orbit-and-index kernels (and the split row gather
+    // where an index allows it): the gather cache is off while it runs, and
+    // its request is restored afterwards
     struct CacheOff {
       GatherCache &gc;
       int saved;
@@ -810,11 +811,13 @@ int spined_operator_autotune(ls_operator *op, int32_t repeats, spined_autotune_r
         std::lock_guard<std::mutex> lk(gc.mu);
         saved = gc.request;
         gc.request = 0;
+        gc.tuning = true;
         gc.drop();
       }
       ~CacheOff() {
         std::lock_guard<std::mutex> lk(gc.mu);
         gc.request = saved;
+        gc.tuning = false;
       }
     } cache_off(*o.cache);
     report->ms_per_matvec_first = time_matvec(o, 1, repeats, x.ptr, y.ptr);
@@ -1091,6 +1094,10 @@ int spined_debug_gather_device(void *dst, uint64_t dst_words, const void *src, u
 }
 
 uint64_t spined_debug_gather_out_words(void) { return gather_calibration_out_words(); }
+
+int spined_debug_matvec_path(const ls_operator *op) {
+  return op && op->p ? op->p->last_path.load() : -1;
+}
 
 int spined_debug_ring_available(const ls_spin_basis *basis) {
   return basis && basis->p->tables.ring_available ? 1 : 0;

@@ -254,6 +254,7 @@ struct GatherCache {
   // locking mu a second time
   std::atomic<bool> building{false};
   int request = -1;       // -1 automatic (built when it fits in free memory), 0 off, 1 on
+  bool tuning = false;    // off for the autotuner: the split row gather stays
   std::atomic<int> calls{0}; // uses of the operator so far (an automatic cache of a small
                              // basis waits for the second)
   bool counted = false;   // classes, woff and total known
@@ -320,6 +321,9 @@ struct Operator {
   // diagonal over the leading low bonds (split.hpp), for the cut of
   // basis->split; built at the first split matvec (under basis->mu)
   mutable DeviceBuffer<double> split_dlow;
+  // kernels of the last matvec (test hook): 0 orbits and index, 1 gather
+  // cache, 2 split row gather; -1 none yet
+  mutable std::atomic<int> last_path{-1};
   std::unique_ptr<GatherCache> cache = std::make_unique<GatherCache>();
   Operator();
   ~Operator();

@@ -1129,8 +1129,9 @@ void launch_split(const Operator &op, const Ctx &c, const XT *x, YT *y, hipStrea
   SPINED_CHECK_LAUNCH();
 }
 
-// Real matvec by the split row gather, unless a gather cache is asked for or
-// several lanes per row are.
+// Real matvec by the split row gather, unless a gather cache is asked for, the
+// orbit kernels are (the cache turned off, other than by the autotuner), or
+// several lanes per row.
 bool try_split(const MatvecCall &m, const Ctx &c) {
   using VT = VecType;
   const Operator &op = *m.op;
@@ -1140,7 +1141,8 @@ bool try_split(const MatvecCall &m, const Ctx &c) {
   if (l < 0 || op.orbit_method() != 0) return false;
   {
     std::lock_guard<std::mutex> lk(op.cache->mu);
-    if (op.cache->request > 0 || op.cache->built) return false;
+    const GatherCache &gc = *op.cache;
+    if (gc.request > 0 || gc.built || (gc.request == 0 && !gc.tuning)) return false;
   }
   Basis &b = *op.basis;
   {
@@ -1335,8 +1337,12 @@ void launch_matvec(const MatvecCall &m) {
     ps = pt.sin_t.ptr;
   }
   const Ctx c = make_ctx(op, pc, ps);
-  if (try_split(m, c)) return;
+  if (try_split(m, c)) {
+    op.last_path = 2;
+    return;
+  }
   const bool done = op.orbit_method() == 1 ? try_cached<1>(m, c) : try_cached<0>(m, c);
+  op.last_path = done ? 1 : 0;
   if (done) return;
   if (op.orbit_method() == 1)
     dispatch<1>(m, c);
@@ -1409,6 +1415,7 @@ void launch_matvec_block(const MatvecBlockCall &m) {
     throw Error(LS_NOT_IMPLEMENTED, "block matvec needs a real operator with <= 256 templates");
   const Ctx c = make_ctx(op, nullptr, nullptr);
   const bool done = op.orbit_method() == 1 ? try_cached_block<1>(m, c) : try_cached_block<0>(m, c);
+  op.last_path = done ? 1 : 0;
   if (done) return;
   if (op.orbit_method() == 1)
     dispatch_block<1>(m, c);

@@ -47,6 +47,7 @@ SPINED_SYMBOLS = (
     "spined_cnn_forward_device", "spined_cnn_backward_device", "spined_cnn_adam_step",
     "spined_cnn_start_vector", "spined_debug_mfma_probe", "spined_debug_copy_device",
     "spined_debug_gather_device", "spined_debug_gather_out_words", "spined_debug_eigh",
+    "spined_debug_matvec_path",
     "spined_batch_eigsh", "spined_operator_autotune",
 )
 
@@ -213,6 +214,7 @@ def load():
         "spined_debug_copy_device": (I, [P, P, U64]),
         "spined_debug_gather_device": (I, [P, U64, P, U64, C.c_int32]),
         "spined_debug_gather_out_words": (U64, []),
+        "spined_debug_matvec_path": (I, [P]),
         "spined_debug_eigh": (I, [C.c_int32, P, P, P]),
     }
     for name, (res, args) in sig.items():

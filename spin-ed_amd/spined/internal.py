@@ -479,6 +479,12 @@ def debug_orbit_hop(basis: SpinBasis, states, sites):
     return reps, ph, cnt, val.astype(bool)
 
 
+def debug_matvec_path(op: Operator_) -> int:
+    """Kernels of the operator's last matvec (test hook): 0 orbits and index, 1
+    gather cache, 2 split row gather; -1 none yet."""
+    return int(_lib.load().spined_debug_matvec_path(op.ptr))
+
+
 def debug_eigh(a):
     """Eigenvalues and eigenvectors (rows) of a symmetric matrix of up to 64
     rows by the eigensolvers' projected-matrix kernel (test hook)."""
