@@ -599,13 +599,17 @@ int resident_blocks() {
 } // namespace
 
 namespace {
-__global__ void __launch_bounds__(kTile) batch_dlow_kernel(const PInst *__restrict__ insts,
-                                                           double *__restrict__ dlow) {
-  const PInst &I = insts[blockIdx.y];
-  const uint32_t e = blockIdx.x * kTile + threadIdx.x;
-  if (I.sp.l > 0 && e < (1u << I.sp.l))
-    dlow[(static_cast<uint64_t>(blockIdx.y) << kSplitLowSites) + e] =
-        split_dlow(I.sp, I.bd, I.sp.lowstate[e]);
+// Diagonal sums (split_dlow) of the instances that take the split row gather,
+// ids[q] into the q-th table (32 KB each).
+constexpr unsigned kDlowBlocks = (1u << kSplitLowSites) / kTile;
+__global__ void __launch_bounds__(kTile)
+    batch_dlow_kernel(const PInst *__restrict__ insts, const uint32_t *__restrict__ ids,
+                      double *__restrict__ dlow) {
+  const uint32_t q = blockIdx.x / kDlowBlocks;
+  const PInst &I = insts[ids[q]];
+  const uint32_t e = (blockIdx.x % kDlowBlocks) * kTile + threadIdx.x;
+  if (e < (1u << I.sp.l))
+    dlow[(static_cast<uint64_t>(q) << kSplitLowSites) + e] = split_dlow(I.sp, I.bd, I.sp.lowstate[e]);
 }
 } // namespace
 
@@ -662,7 +666,7 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
   DeviceBuffer<double> pm(pm_per * n_inst);
   DeviceBuffer<double> outs(8ull * n_inst);
   DeviceBuffer<unsigned> bars(static_cast<uint64_t>(kBarWords) * n_inst);
-  DeviceBuffer<double> dlow(static_cast<uint64_t>(n_inst) << kSplitLowSites);
+  std::vector<uint32_t> split_ids; // instances that take the split row gather
   std::vector<PInst> hinst(n_inst);
   for (int i = 0; i < n_inst; ++i) {
     Operator &op = *ops[i];
@@ -685,7 +689,7 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
     I.out = outs.ptr + 8ull * i;
     I.ntiles = static_cast<uint32_t>((b.D + kTile - 1) / kTile);
     I.sp = SplitArgs{};
-    I.dlow = dlow.ptr + (static_cast<uint64_t>(i) << kSplitLowSites);
+    I.dlow = nullptr;
     I.groups_per_chunk = 1;
     // every site above the low ones counts as high; the top one is down in
     // each row of a flip sector, so it never makes a group of its own
@@ -697,9 +701,13 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
       std::lock_guard<std::mutex> lk(b.mu);
       if (b.split_batch.l < 0) build_split(b, b.split_batch, l);
       I.sp = b.split_args(b.split_batch);
+      if (I.sp.l > 0) split_ids.push_back(static_cast<uint32_t>(i));
       I.groups_per_chunk = static_cast<uint32_t>(std::max<uint64_t>(1, (kChunkTiles * kTile) / std::max<uint64_t>(1, b.D >> nh)));
     }
   }
+  DeviceBuffer<double> dlow(static_cast<uint64_t>(split_ids.size()) << kSplitLowSites);
+  for (size_t q = 0; q < split_ids.size(); ++q)
+    hinst[split_ids[q]].dlow = dlow.ptr + (static_cast<uint64_t>(q) << kSplitLowSites);
   // Team sizes: rows_per_member rows a workgroup, at most max_team of them;
   // when that leaves workgroups without a slot, half the rows and twice the
   // team at a time.  Not up to the last workgroup: every team barrier writes
@@ -735,6 +743,7 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
   const uint32_t nslots = static_cast<uint32_t>(hslots.size());
   DeviceBuffer<PInst> dinst(n_inst);
   DeviceBuffer<Slot> dslots(nslots);
+  DeviceBuffer<uint32_t> dids(split_ids.size());
   SPINED_HIP(hipMemcpyAsync(dinst.ptr, hinst.data(), sizeof(PInst) * n_inst, hipMemcpyHostToDevice, s));
   SPINED_HIP(hipMemcpyAsync(dslots.ptr, hslots.data(), sizeof(Slot) * nslots, hipMemcpyHostToDevice, s));
   DeviceBuffer<unsigned> ticket(1);
@@ -744,9 +753,13 @@ int batch_eigsh(const std::vector<Operator *> &ops, double tol, int m_req, uint6
   batch_init_kernel<<<static_cast<unsigned>((nbar + 255) / 256), 256, 0, s>>>(
       ticket.ptr, abort_flag.ptr, t_start.ptr, bars.ptr, nbar);
   SPINED_CHECK_LAUNCH();
-  batch_dlow_kernel<<<dim3((1 << kSplitLowSites) / kTile, static_cast<unsigned>(n_inst)), kTile, 0, s>>>(
-      dinst.ptr, dlow.ptr);
-  SPINED_CHECK_LAUNCH();
+  if (!split_ids.empty()) {
+    SPINED_HIP(hipMemcpyAsync(dids.ptr, split_ids.data(), 4 * split_ids.size(),
+                              hipMemcpyHostToDevice, s));
+    batch_dlow_kernel<<<static_cast<unsigned>(split_ids.size() * kDlowBlocks), kTile, 0, s>>>(
+        dinst.ptr, dids.ptr, dlow.ptr);
+    SPINED_CHECK_LAUNCH();
+  }
   // one workgroup per slot at most, no more than fit on the device at once
   const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(nslots, static_cast<uint64_t>(resident)));
   SPINED_HIP(hipStreamSynchronize(s));
