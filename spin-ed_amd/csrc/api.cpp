@@ -218,15 +218,21 @@ size_t elem_size(int dtype) {
   }
 }
 
-// Locks the operator's basis for device work: builds are serialised with
-// matvecs, and device tables are uploaded on first use.
+// Device tables are uploaded on first use, by one thread: two uploads of one
+// table would each release the other's block to the pool.
 Operator &prepare_operator(const ls_operator *op) {
   if (!op || !op->p) throw Error(LS_INVALID_ARGUMENT, "operator is NULL");
   Operator &o = *op->p;
   Basis &b = *o.basis;
-  require_built(b);
-  ensure_basis_device(b);
-  ensure_device(o.tables);
+  {
+    std::lock_guard<std::mutex> lk(b.mu);
+    require_built(b);
+    ensure_basis_device(b);
+  }
+  {
+    std::lock_guard<std::mutex> lk(o.mu);
+    ensure_device(o.tables);
+  }
   ensure_schedule(o);
   ++o.cache->calls;
   return o;

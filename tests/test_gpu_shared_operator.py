@@ -53,3 +53,28 @@ def test_threads_share_a_fresh_operator(kind):
             t.join()
         assert not bad
         assert internal.gather_cache(op) == 1 and internal.schedule(op) == 1
+
+
+def test_threads_make_the_first_call_together():
+    """The tables of an operator are uploaded once, whoever comes first."""
+    basis, plain = engine(ring(14, k=0, p=0, z=1))
+    D = internal.get_number_states(basis)
+    X = np.random.default_rng(9).normal(size=(6, D))
+    Y = [spined.apply(plain, x) for x in X]
+    bad = []
+    for round_ in range(40):
+        spec = ring(14, k=0, p=0, z=1)
+        op = spined.mk_operator(basis, [spined.mk_interaction(m, s) for m, s in spec.terms])
+        gate = threading.Barrier(len(X))
+
+        def work(i):
+            gate.wait()
+            if not np.array_equal(spined.apply(op, X[i]), Y[i]):
+                bad.append((round_, i))
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(len(X))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert not bad
