@@ -207,8 +207,10 @@ int spined_operator_get_rows_per_wave(const ls_operator *op);
  * not where the states split into halves that need no entries;
  * given back whenever a device allocation of the library needs the memory),
  * 0 off (the orbit-and-index kernels, also where the states split into
- * halves), 1 on (built at the next matvec; an error if it does not fit).  get:
- * 1 while a cache is built.  Changing the row schedule drops the cache. */
+ * halves), 1 on (built at the next matvec; an error if it does not fit).
+ * Operators of more than 65,535 bonds or templates, or of more than 65,536
+ * products of a coefficient and a character, have none in any mode.  get: 1
+ * while a cache is built.  Changing the row schedule drops the cache. */
 int spined_operator_set_gather_cache(ls_operator *op, int mode);
 int spined_operator_get_gather_cache(const ls_operator *op);
 /* Bucket bits of the bucket index (about 2^bits level-2 buckets of 4 bytes,

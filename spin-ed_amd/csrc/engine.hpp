@@ -257,6 +257,7 @@ struct GatherCache {
   bool tuning = false;    // off for the autotuner: the split row gather stays
   std::atomic<int> calls{0}; // uses of the operator so far (an automatic cache of a small
                              // basis waits for the second)
+  bool unsuitable = false; // more coefficient classes than 16 bits number
   bool counted = false;   // classes, woff and total known
   bool built = false;
   uint64_t total = 0;     // entries

@@ -971,7 +971,7 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
   if (gc.built) return true;
   const Basis &b = *op.basis;
   const int units = unit_count(op.tables);
-  if (gc.request == 0 || b.D > (1ull << 31) || units > 65535) return false;
+  if (gc.request == 0 || gc.unsuitable || b.D > (1ull << 31) || units > 65535) return false;
   // nothing is built under stream capture: its kernels would only run at a replay
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   SPINED_HIP(hipStreamIsCapturing(s, &cap));
@@ -990,8 +990,7 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
   const unsigned g = static_cast<unsigned>(waves);
   if (!gc.counted) {
     if (!cache_classes(op, gc, s)) {
-      if (gc.request > 0)
-        throw Error(LS_NOT_IMPLEMENTED, "gather cache: too many distinct coefficients");
+      gc.unsuitable = true; // also when asked for: as for more than 65,535 units
       return false;
     }
     gc.sched = c.sched;
