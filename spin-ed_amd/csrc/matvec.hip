@@ -989,13 +989,21 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
   const uint64_t waves = (b.D + kRowBlock - 1) / kRowBlock;
   const unsigned g = static_cast<unsigned>(waves);
   if (!gc.counted) {
+    const bool own_sched = !c.sched && schedule_of_cache(op) && op.schedule_request < 0 &&
+                           b.D >= static_cast<uint64_t>(kScheduleTile);
+    // where the reserve is spent no cache can fit: a matvec then needs no
+    // device memory but its vectors, and its tables must not be refused
+    if (gc.request < 0) {
+      size_t free_b = 0, total_b = 0;
+      SPINED_HIP(hipMemGetInfo(&free_b, &total_b));
+      if (free_b < kCacheReserve + (own_sched ? b.D * sizeof(uint16_t) : 0)) return false;
+    }
     if (!cache_classes(op, gc, s)) {
       gc.unsuitable = true; // also when asked for: as for more than 65,535 units
       return false;
     }
     gc.sched = c.sched;
-    if (!gc.sched && schedule_of_cache(op) && op.schedule_request < 0 &&
-        b.D >= static_cast<uint64_t>(kScheduleTile)) {
+    if (own_sched) {
       gc.own_sched.allocate(b.D);
       launch_schedule(op, c, gc.own_sched.ptr, s);
       gc.sched = gc.own_sched.ptr;
