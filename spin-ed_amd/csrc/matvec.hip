@@ -961,6 +961,12 @@ template <int METHOD, class F> void with_fill(const Ctx &c, F &&f) {
     f(std::integral_constant<int, 4>{}, std::false_type{});
 }
 
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  SPINED_HIP(hipStreamIsCapturing(s, &cap));
+  return cap != hipStreamCaptureStatusNone;
+}
+
 // Builds the gather cache when it is requested (1), or when it is automatic
 // (-1), due (see kCacheMinRows; repeated: more matvecs are known to follow)
 // and fits in free memory with kCacheReserve to spare.  Caller holds gc.mu.
@@ -973,9 +979,7 @@ bool ensure_cache(const Operator &op, const Ctx &c, GatherCache &gc, hipStream_t
   const int units = unit_count(op.tables);
   if (gc.request == 0 || gc.unsuitable || b.D > (1ull << 31) || units > 65535) return false;
   // nothing is built under stream capture: its kernels would only run at a replay
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  SPINED_HIP(hipStreamIsCapturing(s, &cap));
-  if (cap != hipStreamCaptureStatusNone) {
+  if (capturing(s)) {
     if (gc.request > 0) throw Error(LS_DEVICE_ERROR, "gather cache: not built under stream capture");
     return false;
   }
@@ -1154,13 +1158,15 @@ bool try_split(const MatvecCall &m, const Ctx &c) {
   Basis &b = *op.basis;
   {
     std::lock_guard<std::mutex> lk(b.mu);
+    // the tables are not built under stream capture either
+    if ((b.split.l < 0 || !op.split_dlow.ptr) && capturing(m.stream)) return false;
     if (b.split.l < 0) {
       if (m.no_alloc) return false;
       build_split(b, b.split, l);
     }
     if (!op.split_dlow.ptr) {
       if (m.no_alloc) return false;
-      // published once it is computed (an error under stream capture)
+      // published once it is computed
       DeviceBuffer<double> d(size_t(1) << l);
       split_dlow_kernel<<<grid_for(uint64_t(1) << l), kBlock, 0, m.stream>>>(
           b.split_args(b.split), c.bd, d.ptr);
