@@ -205,7 +205,8 @@ int spined_operator_get_rows_per_wave(const ls_operator *op);
  * the first matvec of a basis of at least 2^20 rows or of an operator whose
  * matrix-free matvec is long, at the second call or at a solve otherwise;
  * not where the states split into halves that need no entries;
- * given back whenever a device allocation of the library needs the memory),
+ * given back whenever a device allocation of the library needs the memory,
+ * unless a stream capture has recorded a matvec that reads it),
  * 0 off (the orbit-and-index kernels, also where the states split into
  * halves), 1 on (built at the next matvec; an error if it does not fit).
  * Operators of more than 65,535 bonds or templates, or of more than 65,536

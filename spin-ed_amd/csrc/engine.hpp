@@ -260,6 +260,9 @@ struct GatherCache {
   bool unsuitable = false; // more coefficient classes than 16 bits number
   bool counted = false;   // classes, woff and total known
   bool built = false;
+  // a stream capture holds the cache's addresses: it is dropped at the owner's
+  // word only, not for another allocation
+  bool recorded = false;
   uint64_t total = 0;     // entries
   int32_t phases = 1;     // phase classes: 1 (all trivial), 2 (+-1) or L
   int32_t nclass = 0, shift = 0;
@@ -288,7 +291,7 @@ struct GatherCache {
   }
   void drop() {           // caller holds mu
     release_entries();
-    counted = false;
+    counted = recorded = false;
     total = 0;
     sched = nullptr;
     own_sched.release();

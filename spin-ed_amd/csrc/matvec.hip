@@ -1192,6 +1192,7 @@ template <int METHOD> bool try_cached(const MatvecCall &m, const Ctx &c) {
   const bool known = (m.xt == m.yt) || (m.xt == VT::F32 && m.yt == VT::F64);
   if (!known) return false;
   if (m.no_alloc ? !gc.built : !ensure_cache<METHOD>(*m.op, c, gc, m.stream)) return false;
+  if (!gc.recorded && capturing(m.stream)) gc.recorded = true;
   const bool order = contiguous_rows(*m.op, m.xt == VT::F32);
   if (m.xt == VT::F64)
     launch_cached<RealRows<double, double, 1>>(*m.op, c, gc, m.x, m.y, order, m.stream);
@@ -1263,6 +1264,7 @@ template <int METHOD> bool try_cached_block(const MatvecBlockCall &m, const Ctx 
   const bool f32 = m.xt == VT::F32 && (m.yt == VT::F32 || m.yt == VT::F64);
   if (!f64 && !f32) return false;
   if (!ensure_cache<METHOD>(*m.op, c, gc, m.stream)) return false;
+  if (!gc.recorded && capturing(m.stream)) gc.recorded = true;
   if (f64)
     launch_cached_rows<double, double>(m, c, gc);
   else if (m.yt == VT::F32)
@@ -1382,7 +1384,7 @@ bool prepare_gather_cache(Operator &op, uint64_t reserve, uint64_t block_bytes) 
 
 void drop_gather_cache_if_built(Operator &op) {
   std::lock_guard<std::mutex> lk(op.cache->mu);
-  if (op.cache->built) op.cache->release_entries();
+  if (op.cache->built && !op.cache->recorded) op.cache->release_entries();
 }
 
 Operator::Operator() {
@@ -1400,14 +1402,14 @@ void drop_gather_cache(Operator &op) {
   op.cache->drop();
 }
 
-// Caches in use (their lock held) are left alone.
+// Caches in use (their lock held) or recorded in a graph are left alone.
 void reclaim_gather_caches(int device) {
   std::lock_guard<std::mutex> lk(g_ops_mu);
   for (Operator *op : g_ops) {
     if (!op->basis || op->basis->device != device) continue;
     GatherCache &gc = *op->cache;
     if (gc.building.load() || !gc.mu.try_lock()) continue;
-    if (gc.built) gc.release_entries();
+    if (gc.built && !gc.recorded) gc.release_entries();
     gc.mu.unlock();
   }
 }
