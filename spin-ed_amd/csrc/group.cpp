@@ -249,10 +249,13 @@ void detect_torus(const Group &g, int n, OrbitTables &t) {
   }
 }
 
+// The callers wait once for all tables of an object (`h` is a member of it;
+// a wait for each of fifteen tables made the first complex matvec of 9,252 rows
+// 304 us instead of 175).
 template <class T> void upload(DeviceBuffer<T> &d, const std::vector<T> &h) {
   d.allocate(std::max<size_t>(h.size(), 1));
   if (!h.empty())
-    copy_in(d.ptr, h.data(), h.size() * sizeof(T));
+    SPINED_HIP(hipMemcpyAsync(d.ptr, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, stream()));
 }
 } // namespace
 
@@ -368,6 +371,7 @@ void ensure_device(OrbitTables &t) {
   upload(t.row_key, t.h_row_key);
   upload(t.div_idx, t.h_div_idx);
   upload(t.ratio, t.h_ratio);
+  SPINED_HIP(hipStreamSynchronize(stream()));
   t.on_device = true;
 }
 
@@ -574,6 +578,7 @@ void ensure_device(OperatorTables &t) {
   upload(t.bond_o, t.h_bond_o);
   upload(t.bond_flip, t.h_bond_flip);
   upload(t.bond_lo, t.h_bond_lo);
+  SPINED_HIP(hipStreamSynchronize(stream()));
   t.on_device = true;
 }
 
