@@ -85,9 +85,10 @@ typedef struct spined_eigsh_options {
 } spined_eigsh_options;
 
 typedef struct spined_stats {
-  int64_t matvecs;          /* total H*v applications.  Sectors below 2^20 rows may take
-                             * up to one cycle more than the convergence needs: far
-                             * from it the estimates are looked at between cycles only */
+  int64_t matvecs;          /* total H*v applications.  In sectors of 4,096 to 2^20 rows
+                             * a start vector of a few eigenvectors may take up to one
+                             * cycle more than its convergence needs: far from it the
+                             * estimates are looked at between cycles only */
   int64_t matvecs_mixed;    /* of which in the FP32-storage phase */
   int32_t restarts;
   double seconds_total;

@@ -854,18 +854,20 @@ template <class VT, bool C = false> struct Phase {
     // Convergence is also checked inside a cycle (on the leading block of T)
     // so that a good start vector is not held back to a restart boundary:
     // every step when a matvec is expensive, every 4th otherwise.  There a
-    // check is as long as three steps, and after one that finds the estimate
-    // more than kFarEstimate from the target the next is the cycle's last: a
-    // solve gains about a factor 10 in four steps, so it sees its convergence
-    // at the step where a check every fourth step would (the same matvecs in
-    // 24 solves of sectors of 85 to 101,340 rows; four levels of the 24-site
-    // ring 5.6 ms, 6.6 with every fourth step checked, 6.2 with a wait of four
-    // steps for every factor kFarEstimate).  A start vector of a few
-    // eigenvectors exhausts its Krylov space within the cycle; such a solve
-    // goes on to the cycle's end, and the steps after its breakdown, which is
-    // read with the check, are taken again.
+    // check is as long as three steps, and from kFarCheckRows rows on, after one
+    // that finds the estimate more than kFarEstimate from the target, the next
+    // is the cycle's last: four steps gain about a factor 10 (four levels of the
+    // 24-site ring 5.6 ms, 6.6 with every fourth step checked).  Only where the
+    // Krylov space comes near its end do they gain kFarEstimate: of 927 solves of
+    // sectors of 76 to 26,500 rows, 48 took 4 to 12 matvecs more without the
+    // checks, all below 1,300 rows; from 4,096 rows on none did.  (A start
+    // vector of a few eigenvectors comes to that end in any sector; in a large
+    // one it goes on to the end of the cycle.)  The steps after a breakdown,
+    // which is read with the check, are taken again.
     const int check_every = n >= (1u << 20) ? 1 : 4;
     constexpr double kFarEstimate = 1e5;
+    constexpr uint64_t kFarCheckRows = 4096;
+    const bool every_check = check_every == 1 || n < kFarCheckRows;
     int checked = 0; // steps whose breakdown flag has been read
     // Solves the leading msz x msz projected problem; estimates of the k
     // lowest.  Returns the first unchecked step that broke down before the
@@ -910,7 +912,7 @@ template <class VT, bool C = false> struct Phase {
         step(j);
         const int msz = j + 1;
         const bool check = msz < m && msz > k && (msz - j0) % check_every == 0 &&
-                           (check_every == 1 || near <= kFarEstimate * tol);
+                           (every_check || near <= kFarEstimate * tol);
         if (!check && msz < m) continue;
         const int broke = project(msz, worst, nconv);
         if (broke >= 0) {
