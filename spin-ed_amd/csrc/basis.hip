@@ -61,12 +61,15 @@ __device__ inline uint64_t next_state(const EnumArgs &e, uint64_t v) {
   return (t + 1) | (((~t & (0 - ~t)) - 1) >> (__builtin_ctzll(v) + 1));
 }
 
+// METHOD: 0 generic, 1 ring, 2 torus with row keys.
 template <int METHOD>
 __device__ inline bool is_basis_state(const GenericOrbitArgs &ga, const RingOrbitArgs &ra,
                                       uint64_t x) {
   if constexpr (METHOD == 1) {
     const OrbitResult r = orbit_ring(ra, x);
     return r.rep == x && r.valid;
+  } else if constexpr (METHOD == 2) {
+    return rep_test_torus_key(ga, x) != 0;
   } else {
     return rep_test_generic(ga, x) != 0;
   }
@@ -541,6 +544,8 @@ void build_basis(Basis &b) {
     const unsigned nb = grid_for(nw);
     if (b.tables.ring_available)
       enumerate_kernel<1><<<nb, kBlock, 0, s>>>(e, ga, ra, w0, nw, masks.ptr, counts.ptr);
+    else if (ga.row_key)
+      enumerate_kernel<2><<<nb, kBlock, 0, s>>>(e, ga, ra, w0, nw, masks.ptr, counts.ptr);
     else
       enumerate_kernel<0><<<nb, kBlock, 0, s>>>(e, ga, ra, w0, nw, masks.ptr, counts.ptr);
     SPINED_CHECK_LAUNCH();

@@ -208,7 +208,8 @@ __host__ __device__ inline uint64_t orbit_min_torus_key(const GenericOrbitArgs &
   return best;
 }
 
-// rep_test_generic by row keys: x fails as soon as some row's key is below
+// rep_test_generic by row keys (a kernel of its own takes it: in one with the
+// scans its registers cost every other group a wave per SIMD): x fails as soon as some row's key is below
 // x's own top row.
 __host__ __device__ inline uint32_t rep_test_torus_key(const GenericOrbitArgs &a, uint64_t x) {
   const uint32_t top = static_cast<uint32_t>(x >> (a.n_sites - a.torus_l1));
@@ -345,7 +346,6 @@ __host__ __device__ inline uint64_t orbit_min_generic(const GenericOrbitArgs &a,
 // else 0.
 // rep_test_generic over the torus factorisation (same result).
 __host__ __device__ inline uint32_t rep_test_torus(const GenericOrbitArgs &a, uint64_t x) {
-  if (a.row_key) return rep_test_torus_key(a, x);
   const uint64_t rx = reverse_n(x, a.n_sites);
   const int l1 = a.torus_l1, l2 = a.torus_l2, n = a.n_sites;
   const uint64_t mask = a.site_mask;
