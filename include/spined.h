@@ -198,7 +198,7 @@ int spined_operator_get_schedule(const ls_operator *op);
 int spined_operator_set_rows_per_wave(ls_operator *op, int rows);
 int spined_operator_get_rows_per_wave(const ls_operator *op);
 /* Gather cache of an operator: the target of every term of every row (4
- * bytes per term and 10 per row, padded per wave: ~81 GB at D = 8.6e8),
+ * bytes per term and 10 per row, padded per wave: ~83 GB at D = 8.6e8),
  * written once by the orbit and index kernels so that later matvecs read it
  * instead of recomputing orbits and searching the index; the sums are
  * identical.

@@ -206,7 +206,7 @@ __device__ inline double broke_down(double beta, double tjj) {
   return beta <= 1e-12 * fmax(1.0, fabs(tjj)) ? 1.0 : 0.0;
 }
 // The second Gram-Schmidt pass runs only when the first update keeps less
-// than this fraction of |w| (second_pass_test_kernel).
+// than this fraction of |w| (first_pass_kernel).
 constexpr double kSecondPassEta = 1e-2;
 constexpr int64_t kAutoMaxMatvecs = 20000; // spined_eigsh_options.max_matvecs = 0
 
